@@ -25,21 +25,27 @@ __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu
                       unsigned* next_task, apk_tile_record* log) {
   __shared__ __attribute__((aligned(16))) char ring[E::LDS_BYTES];
   __shared__ unsigned s_task;
+  __shared__ proto::QueueCursor s_cur;  // thread 0's place in the queue
 
   const int tilesN = N / E::TN;
   const unsigned numTasks = (unsigned)((M / E::TM) * tilesN);
-  const TaskQueue tq(next_task, M / E::TM, tilesN, numTasks);
+  // The launch owns its counters: every worker's first task is fixed.
+  const TaskQueue tq(next_task, M / E::TM, tilesN, numTasks, gridDim.x);
   const int home = (int)xcc_id();
   const int nChunks = K / kChunk;
   const int spc = kChunk / E::KS;  // k-stages per chunk
   const typename E::Ctx ctx = E::make_ctx(A, B, M, N, K);
   const uint32_t wl = wave_lds(ring);
+  if (threadIdx.x == 0) {
+    s_cur = proto::QueueCursor{0, 0, 0, 0, 0};
+    tq.start(s_cur, blockIdx.x);
+  }
 
   for (;;) {
     // Reconverge before the thread-0 pop (no thread-0 region of the previous
     // iteration may be threaded into this one across the back-edge).
     lds_sync();
-    if (threadIdx.x == 0) s_task = tq.pop(home);
+    if (threadIdx.x == 0) s_task = tq.pop(home, s_cur);
     __syncthreads();
     const unsigned task = uniform(s_task);
     __syncthreads();  // every thread has read s_task before it is rewritten
@@ -80,6 +86,13 @@ __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu
       rec[nChunks - 1].block = (int)blockIdx.x;
     }
   }
+  // The counters end as if every worker had taken its first task from them
+  // and failed once on every list: one block adds that for all, with one
+  // request, after the last task is handed out.
+  if (blockIdx.x == 0 && threadIdx.x < APK_QUEUE_XCDS && tq.list_total((int)threadIdx.x) > 0)
+    __hip_atomic_fetch_add(&next_task[threadIdx.x],
+                           gridDim.x + tq.list_first((int)threadIdx.x), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The urgent job as the reference runs it (urgent_tile, src/urgent_baseline.cu:

@@ -57,6 +57,7 @@ k_persistent_yield(const apk_yield_params) {
   __shared__ long long s_setter[2];  // next event, time base
   __shared__ long long s_serve_t1;   // start of the current service's urgent work
   __shared__ int s_fsync;            // synchronous flag read (syncPoll)
+  __shared__ proto::QueueCursor s_cur;  // thread 0's place in the work queue
 
   const int tid = threadIdx.x, bid = blockIdx.x;
   // Values the stage loop does not need are recomputed from the parameters
@@ -84,6 +85,16 @@ k_persistent_yield(const apk_yield_params) {
     return (st + E::GROUP - 1) / E::GROUP * E::GROUP;
   }();
   int chunksDone = 0;  // uniform
+  // Tasks taken per pop. A grid of W workers makes W pops per task time, and
+  // the queue serves one per 12 ns (protocol.hpp): tasks of a few k-stages are
+  // taken several at a time. Longer ones singly, so that the tiles in flight
+  // stay next to each other in the grid and share panels in L2. A block of the
+  // retreat arm takes one at a time: it may leave at any site, and must not
+  // hold tasks that it has not begun.
+  auto popBatch = [&]() -> unsigned {
+    const int stages = P().K / E::KS;
+    return RETREAT || stages >= 16 ? 1u : (unsigned)(16 / stages);
+  };
   const i32x4 flag_rsrc =
       make_rsrc((const char*)P().flag + (size_t)(bid % copies()) * APK_FLAG_STRIDE, 4);
   const bool isSetter = P().flag_set != nullptr && P().sched != nullptr && bid == 0;
@@ -119,6 +130,7 @@ k_persistent_yield(const apk_yield_params) {
   if (tid <= E::NS) flagring[tid] = 0;
   if (tid < APK_STATS_PER_BLOCK) s_stats[tid] = 0;
   if (tid < 2) s_setter[tid] = 0;
+  if (tid == 0) s_cur = proto::QueueCursor{0, 0, 0, 0, 0};
   if (P().run_gt && bid == 0 && tid == 0) P().run_gt[0] = wall_ticks();
   __syncthreads();
   if constexpr (retreatArm) {
@@ -194,7 +206,14 @@ k_persistent_yield(const apk_yield_params) {
   int savedKind = FRESH;
 
   for (;;) {
-    if (POLL != APK_POLL_OFF && serving < 0 && fLatest < 0) break;  // host stop sentinel
+    // host stop sentinel: no task is taken any more (one taken with an
+    // earlier pop is still run)
+    if (POLL != APK_POLL_OFF && serving < 0 && fLatest < 0) {
+      lds_sync();
+      const unsigned held = uniform(s_cur.end - s_cur.next);
+      lds_sync();
+      if (held == 0) break;
+    }
     // Reconverge before the thread-0 pop: without a barrier here the
     // compiler may thread the previous iteration's thread-0 regions into
     // this one across the back-edge and split the block's lanes over two
@@ -269,7 +288,8 @@ k_persistent_yield(const apk_yield_params) {
           // the task-start sample goes out in front of the pop's fetch-add,
           // and the wait for the pop retires it
           if (startSites) sample_flag<SYS>(flag_rsrc, flag_lds + 4u * (uint32_t)E::NS);
-          t = TaskQueue(P().next_task, P().M / E::TM, tilesN(), P().num_tasks).pop((int)xcc_id());
+          t = TaskQueue(P().next_task, P().M / E::TM, tilesN(), P().num_tasks)
+                  .pop((int)xcc_id(), s_cur, popBatch(), gridDim.x);
           if (startSites) wait_vmcnt<0>();
         }
         s_u32 = t;

@@ -43,16 +43,37 @@ namespace proto {
 // (counter ctr[q]) and, once that is exhausted, the other lists in turn, so
 // every task id below num_tasks is handed out exactly once and task u always
 // computes tile u % T.
+//
+// What bounds it: the eight counters lie in one 64-byte line, and the device
+// serves about 85 M atomics/s on one line, whoever sends them (12 ns each;
+// 200,000 two-stage tasks took 2.43 ms, 1.94 ms with the rules below). So a
+// worker spares the line where it can:
+//  - a list it has found exhausted it never tries again, and on finding one
+//    it reads all eight counters at once instead of trying the other lists
+//    one atomic at a time (with 1024 workers those 8 failing atomics each
+//    were most of the 111 us of a 221-tile GEMM; now 28 us);
+//  - short tasks are taken several at a time (`batch`), fewer as the list
+//    runs out;
+//  - `statics` > 0 (a launch that owns its counters): worker b starts with
+//    position b / 8 of list b % 8, no atomic at all, and the counters hand
+//    out the positions after those.
+constexpr unsigned TQ_NONE = 0xffffffffu;
+// One worker's place in the queue: positions [next, end) of `list` are its
+// own; bit q of `dead` marks list q exhausted; `seen` is the last index its
+// own list's counter gave it. All zero at the start.
+struct QueueCursor {
+  unsigned next, end, list, dead, seen;
+};
 template <class P>
 struct TaskQueue {
   static constexpr int GM = 4;
   unsigned* ctr;
   int tilesM, tilesN, T;
-  unsigned numTasks, passes;
+  unsigned numTasks, passes, statics;
 
-  APK_PROTO_FN TaskQueue(unsigned* c, int tm, int tn, unsigned n)
+  APK_PROTO_FN TaskQueue(unsigned* c, int tm, int tn, unsigned n, unsigned st = 0)
       : ctr(c), tilesM(tm), tilesN(tn), T(tm * tn), numTasks(n),
-        passes((n + (unsigned)(tm * tn) - 1) / (unsigned)(tm * tn)) {}
+        passes((n + (unsigned)(tm * tn) - 1) / (unsigned)(tm * tn)), statics(st) {}
 
   APK_PROTO_FN int grouped(int i) const {
     const int band = i / (GM * tilesN);
@@ -64,23 +85,73 @@ struct TaskQueue {
   APK_PROTO_FN int list_begin(int q) const {
     return (int)(((long long)q * T) / APK_QUEUE_XCDS);
   }
-  // One caller per block. Returns the next task id, or 0xffffffff when every
-  // list is exhausted.
-  APK_PROTO_FN unsigned pop(int home) const {
-    for (int k = 0; k < APK_QUEUE_XCDS; ++k) {
-      const int q = (home + k) & (APK_QUEUE_XCDS - 1);
-      const int b = list_begin(q), n = list_begin(q + 1) - b;
-      if (n == 0) continue;
-      const unsigned total = (unsigned)n * passes;
-      for (;;) {
-        const unsigned j = P::fetch_add(&ctr[q], 1u);
-        if (j >= total) break;
+  // Positions of list q over all passes, and how many of them are the
+  // workers' first tasks.
+  APK_PROTO_FN unsigned list_total(int q) const {
+    return (unsigned)(list_begin(q + 1) - list_begin(q)) * passes;
+  }
+  APK_PROTO_FN unsigned list_first(int q) const {
+    const unsigned w = (statics + APK_QUEUE_XCDS - 1 - (unsigned)q) / APK_QUEUE_XCDS;
+    const unsigned total = list_total(q);
+    return w < total ? w : total;
+  }
+  // Worker b's first task (statics > b): nothing if its list is shorter.
+  APK_PROTO_FN void start(QueueCursor& c, unsigned b) const {
+    c.list = b % APK_QUEUE_XCDS;
+    c.next = b / APK_QUEUE_XCDS;
+    c.end = c.next < list_first((int)c.list) ? c.next + 1 : c.next;
+  }
+  // One caller per block. Returns the next task id, or TQ_NONE when every
+  // list is exhausted. `batch` > 1: up to that many consecutive positions of
+  // the worker's own list per atomic, while at least 8 batches per worker of
+  // the list (`workers` in all) are left by the last index seen.
+  APK_PROTO_FN unsigned pop(int home, QueueCursor& cursor, unsigned batch = 1,
+                            unsigned workers = 1) const {
+    QueueCursor c = cursor;  // one read and one write of the caller's (LDS) copy
+    const unsigned u = pop_local(home, c, batch, workers);
+    cursor = c;
+    return u;
+  }
+  APK_PROTO_FN unsigned pop_local(int home, QueueCursor& c, unsigned batch,
+                                  unsigned workers) const {
+    for (;;) {
+      if (c.next < c.end) {
+        const int b = list_begin((int)c.list);
+        const unsigned n = (unsigned)(list_begin((int)c.list + 1) - b), j = c.next++;
         const unsigned u =
-            (j / (unsigned)n) * (unsigned)T + (unsigned)grouped(b + (int)(j % (unsigned)n));
+            (j / n) * (unsigned)T + (unsigned)grouped(b + (int)(j % n));
         if (u < numTasks) return u;
+        continue;
       }
+      int k = 0;
+      if (c.dead) {
+        while (k < APK_QUEUE_XCDS && (c.dead >> ((home + k) & (APK_QUEUE_XCDS - 1)) & 1u)) ++k;
+        if (k == APK_QUEUE_XCDS) return TQ_NONE;
+      }
+      const int q = (home + k) & (APK_QUEUE_XCDS - 1);
+      const unsigned first = list_first(q), total = list_total(q) - first;
+      unsigned take = 1;
+      if (k == 0 && batch > 1) {
+        const unsigned each = (total - c.seen) / (workers + APK_QUEUE_XCDS - 1);
+        take = each < 1 ? 1 : each < batch ? each : batch;
+      }
+      unsigned j = total;
+      if (total > 0) j = P::fetch_add(&ctr[q], take);
+      if (j < total) {
+        if (k == 0) c.seen = j;
+        c.list = (unsigned)q;
+        c.next = first + j;
+        c.end = first + (total - j < take ? total : j + take);
+        continue;
+      }
+      // Exhausted: look at all the counters in one round trip. A counter
+      // only grows, so a list seen exhausted stays so.
+      c.dead |= 1u << q;
+      unsigned v[APK_QUEUE_XCDS];
+      for (int i = 0; i < APK_QUEUE_XCDS; ++i) v[i] = P::load(&ctr[i]);
+      for (int i = 0; i < APK_QUEUE_XCDS; ++i)
+        if (v[i] >= list_total(i) - list_first(i)) c.dead |= 1u << i;
     }
-    return 0xffffffffu;
   }
 };
 

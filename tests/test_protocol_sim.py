@@ -195,3 +195,22 @@ def test_retreat_short_ring_waits(seed):
                                "--retreat", 6, "--domains", 6, "--cap", 2, "--seed", seed,
                                "--rq-wait-us", 2000, cover=refused, attempts=8)
     assert f["stuck"] == 0 and f["lost"] == 0, line
+
+
+@pytest.mark.parametrize("batch", [1, 3, 8])
+@pytest.mark.parametrize("statics", [0, 1])
+@pytest.mark.parametrize("blocks,tiles_m,tiles_n,passes", [
+    (16, 1, 1, 1),    # one tile: seven empty lists
+    (3, 3, 2, 1),     # fewer workers than lists, fewer tiles than lists
+    (13, 5, 9, 3),    # lists of unequal length, steals between them
+    (16, 2, 4, 1),    # one position per list
+    (16, 16, 16, 16), # batches shrink as the lists run out
+])
+def test_queue_hands_out_every_task_once(batch, statics, blocks, tiles_m, tiles_n, passes):
+    """Several tasks per pop and fixed first tasks, over list lengths from
+    zero up: every task done exactly once."""
+    rc, line, f = run("--arm", "coop", "--blocks", blocks, "--tiles-m", tiles_m, "--tiles-n",
+                      tiles_n, "--passes", passes, "--stages", 2, "--work-ns", 200, "--events", 3,
+                      "--batch", batch, "--statics", statics, job=False)
+    assert rc == 0 and line.startswith("PASS"), line
+    assert f["dup"] == 0 and f["miss"] == 0, line
