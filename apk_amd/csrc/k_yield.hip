@@ -24,6 +24,8 @@
 // Every branch that contains a barrier is taken on values all threads read
 // from LDS after a barrier (the snapshot discipline of src/midyield.cu:
 // 177-200), so a block never splits across barriers.
+#include <climits>
+
 #include "capi.hpp"
 #include "engine_bf16.hpp"
 #include "engine_mfma128.hpp"
@@ -54,7 +56,8 @@ k_persistent_yield(const apk_yield_params) {
   // Block-wide counters of thread 0 (yields, times, retreats, ...) and the
   // setter's state live in LDS: they are touched only off the stage loop.
   __shared__ unsigned long long s_stats[APK_STATS_PER_BLOCK];
-  __shared__ long long s_setter[2];  // next event, time base
+  __shared__ long long s_setter[3];  // next event, time base, when it is due
+  __shared__ int s_due[2];           // due, as of the setter's last site / this one
   __shared__ long long s_serve_t1;   // start of the current service's urgent work
   __shared__ int s_fsync;            // synchronous flag read (syncPoll)
   __shared__ proto::QueueCursor s_cur;  // thread 0's place in the work queue
@@ -129,7 +132,8 @@ k_persistent_yield(const apk_yield_params) {
   const uint32_t flag_lds = lds_addr_of(flagring);
   if (tid <= E::NS) flagring[tid] = 0;
   if (tid < APK_STATS_PER_BLOCK) s_stats[tid] = 0;
-  if (tid < 2) s_setter[tid] = 0;
+  if (tid < 3) s_setter[tid] = 0;
+  if (tid < 2) s_due[tid] = 1;  // the first site sets the time base
   if (tid == 0) s_cur = proto::QueueCursor{0, 0, 0, 0, 0};
   if (P().run_gt && bid == 0 && tid == 0) P().run_gt[0] = wall_ticks();
   __syncthreads();
@@ -174,6 +178,20 @@ k_persistent_yield(const apk_yield_params) {
   auto set_flag = [&](int v) {
     for (int c = 0, n = copies(); c < n; ++c)
       flag_store((int*)((char*)P().flag_set + (size_t)c * APK_FLAG_STRIDE), v);
+  };
+
+  // Whether the setter has something to do at this site (uniform; called
+  // once per site, after a barrier): thread 0 looked at the clock at the last
+  // one, and looks again now for the next. The block leaves the stage loop
+  // only then, not at every site: leaving drains the software pipeline, which
+  // would make the setter's tiles the slowest of the grid.
+  int dueSite = 0;  // uniform
+  auto setter_due = [&]() -> bool {
+    if (!isSetter) return false;
+    const bool due = uniform(s_due[dueSite]) != 0;
+    dueSite ^= 1;
+    if (tid == 0) s_due[dueSite] = wall_ticks() >= s_setter[2];
+    return due;
   };
 
   // Broadcast a value thread 0 computed (uniform afterwards).
@@ -509,7 +527,7 @@ k_persistent_yield(const apk_yield_params) {
                 f = uniform(s_fsync);
               }
               fLatest = f;
-              if (f != lastSeen || isSetter) {
+              if ((int)setter_due() | (f != lastSeen)) {
                 fSeen = f;
                 atSite = true;
                 ahead = POLL == APK_POLL_ISSUE;
@@ -552,7 +570,7 @@ k_persistent_yield(const apk_yield_params) {
               f = uniform(s_fsync);
             }
             fLatest = f;
-            if (f != lastSeen || isSetter) {
+            if ((int)setter_due() | (f != lastSeen)) {
               fSeen = f;
               atSite = true;
               return false;
@@ -616,17 +634,30 @@ k_persistent_yield(const apk_yield_params) {
         if (s_setter[1] == 0) s_setter[1] = now;
         const long long gBase = s_setter[1];
         const int nextEv = (int)s_setter[0];
-        if (nextEv < P().num_events) {
-          if (now >= gBase + P().sched[nextEv]) {
-            P().set_gt[nextEv] = now;
-            s_setter[0] = nextEv + 1;
-            set_flag(nextEv + 1);
+        // An event is raised only where this block has a later site to see it
+        // from (a flag store shows up in its own samples two or three stages
+        // later): raised at the end of the job's last tile, nobody would be
+        // left to serve it. So at a tile's end it waits unless tasks are left.
+        const int margin = pollStride > 4 ? pollStride : 4;
+        const bool room =
+            S <= 2 * margin || s + margin < S ||
+            TaskQueue(P().next_task, P().M / E::TM, tilesN(), P().num_tasks).any_left();
+        const long long stopAt =
+            gBase + (P().num_events ? P().sched[P().num_events - 1] : 0) + P().stop_after;
+        int ev = nextEv;
+        if (ev < P().num_events) {
+          if (room && now >= gBase + P().sched[ev]) {
+            P().set_gt[ev] = now;
+            set_flag(++ev);
+            s_setter[0] = ev;
           }
-        } else if (P().stop_after > 0 &&
-                   now >= gBase + (P().num_events ? P().sched[P().num_events - 1] : 0) +
-                              P().stop_after) {
+        } else if (P().stop_after > 0 && now >= stopAt) {
           set_flag(-1);  // self-terminating run: no host in the loop
         }
+        const long long at = ev < P().num_events ? gBase + P().sched[ev]
+                             : P().stop_after > 0 ? stopAt : LLONG_MAX;
+        s_setter[2] = at;
+        s_due[0] = s_due[1] = now >= at;
       }
       if (f > P().num_events) f = P().num_events;  // never index past the event arrays
       srcKind = AS_IS;

@@ -95,6 +95,12 @@ struct TaskQueue {
     const unsigned total = list_total(q);
     return w < total ? w : total;
   }
+  // Whether any position is still to be handed out.
+  APK_PROTO_FN bool any_left() const {
+    for (int q = 0; q < APK_QUEUE_XCDS; ++q)
+      if (P::load(&ctr[q]) < list_total(q) - list_first(q)) return true;
+    return false;
+  }
   // Worker b's first task (statics > b): nothing if its list is shorter.
   APK_PROTO_FN void start(QueueCursor& c, unsigned b) const {
     c.list = b % APK_QUEUE_XCDS;
