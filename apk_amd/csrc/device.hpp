@@ -128,6 +128,8 @@ __device__ __forceinline__ float4 buf_load_f4(buf_rsrc r, int voff, int soff) {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // splitmix64 finaliser: the mixing step of the tile fingerprints.
 __device__ __forceinline__ uint64_t mix64(uint64_t z) {

@@ -80,8 +80,6 @@
 
 namespace apk {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
 template <int TM_, int TN_, int THREADS_, int BPC_, int KS_, int IVMAX_>
 struct EngBf16T {
   static_assert(TM_ == 128 || TM_ == 256, "128 or 256 tile rows");
@@ -407,7 +405,7 @@ struct EngBf16T {
     return true;
   }
   // The last pair's deferred MFMAs, before the accumulators are read.
-  static __device__ __forceinline__ void finish_tail(Acc& acc, const Tail& tail) {
+  static __device__ __forceinline__ void finish_tail(const char*, Acc& acc, const Tail& tail) {
 #pragma unroll
     for (int m = 0; m < NT_MF; ++m) {
       const int rb = m / CB, cb = m % CB;

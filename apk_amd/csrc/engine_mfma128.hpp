@@ -1,25 +1,39 @@
-// engine_mfma128.hpp -- 128x128 fp32 output tile on the gfx950 fp32 matrix
-// cores (v_mfma_f32_32x32x2_f32), fed by a 3-stage LDS ring of
-// buffer_load_dwordx4 ... lds (direct-to-LDS, no VGPR staging).
+// engine_mfma128.hpp -- 128x128 fp32 output tile on the gfx950 matrix cores,
+// fed by a 3-stage LDS ring of buffer_load_dwordx4 ... lds (direct-to-LDS, no
+// VGPR staging).
 //
-// Two ring shapes of the same tile (template parameter G):
-//  G = 1 (EngMfma128): 3 slots, one barrier per k-stage -- the preemptible
-//        kernels, which poll at every k-stage;
-//  G = 2 (EngMfma128Pairs): 4 slots (128 KiB) taken in pairs of k-stages,
-//        one barrier per pair -- the non-preemptible persistent GEMM and the
-//        urgent-job kernel, for tiles of an even number of k-stages. With
-//        one wave per SIMD nothing covers a barrier's wait and first operand
-//        reads, so halving the barriers gains 1.5-2% (4096^3 and 8192^3,
-//        ABAB).
-// Both walk every output's k in the same order, so their C is bit-identical.
+// The fp32 matrix instructions give 157 TFLOP/s, the bf16 ones sixteen times
+// that. Each operand is therefore split into three bf16 parts, x = hi + mid +
+// lo, every part the round-to-nearest bf16 of what the former leave: 24
+// significand bits in all, so x is represented exactly. A product is the sum
+// of the six part products down to 2^-16 of hi.hi (the three left out are
+// below 2^-24 of it), accumulated in fp32 by v_mfma_f32_32x32x16_bf16, which
+// rounds once per 8 products where the fp32 instructions round at every one.
+// Error against 64 bits, uniform [-1, 1) operands, K = 256 / 992 / 4096:
+// 2.3e-7 / 4.8e-7 / 1.0e-6 (fp32 chain 2.9e-7 / 5.6e-7 / 1.1e-6).
+// What the parts cannot carry is computed with exact fp32 products instead
+// (suspect, compute_exact): tiles with an infinite or NaN accumulator (an
+// operand or a sum that is infinite, NaN, or above bf16's largest value) and
+// tiles with an operand below 2^-100 other than zero (its lowest part could
+// be rounded).
 //
 // Block: 256 threads = 4 wave64s in a 2x2 arrangement; each wave owns a
 // 64x64 sub-tile held as 2x2 32x32 accumulators (64 VGPRs per lane).
 // Stage: k depth KS=32 -> A stage 128x32 fp32 (16 KiB) + B stage 32x128 fp32
-// (16 KiB); 3 stages = 96 KiB (pairs: 4 = 128 KiB) of the 160 KiB LDS (1 block
-// per CU).
+// (16 KiB); 3 stages = 96 KiB of the 160 KiB LDS, and 48 KiB of split operands
+// (planes): 1 block per CU.
 //
-// LDS layouts (bank-conflict-free for the MFMA operand reads):
+// What bounds it: a 16-deep k-step is 24 MFMAs per wave (768 matrix cycles)
+// and, with each operand split once per block, 16 values per lane to split
+// (6.5 vector instructions each). At 4096^3 it takes about 1.75 K cycles at
+// 2.25 GHz: a wave issues in order, one per SIMD, and meets the LDS traffic of
+// the planes (18 instructions per wave and step); without them 1.2 K, at 2.0
+// GHz (the package then limits the clock). Splitting in every wave for itself
+// (no planes, twice the vector work) is no faster, and 6% slower with polls.
+// 4096^3: 970 -> 800 us; 1920x1408x992: 67 -> 53; 8192x8192x4096 with
+// chunk polls: 4130 -> 3430.
+//
+// LDS layouts (bank-conflict-free):
 //  A stage: 128 rows x 128 B. 16-byte quad q of row r is stored at slot
 //           q ^ aswz(r), aswz(r) = (r ^ ((r >> 3) & 1)) & 7: 8 (or 16)
 //           consecutive rows reading the same quad hit 8 (16) different
@@ -31,33 +45,36 @@
 //           upper one; the XOR moves the upper half by 128 B, so the two
 //           halves never share a bank even when all 64 lanes are served in
 //           one cycle.
+//  planes:  a k-step's split operands, per 32-row block (0-3 of A, 4-7 of B)
+//           and part 64 lanes x 16 B, in the lane order of the MFMA operand:
+//           written and read by whole waves at 16 bytes per lane.
 //
-// k order inside a stage: k-group g (8 values) is consumed in 4 MFMA steps;
-// in step s the lower half-wave supplies k = 8g+s and the upper half-wave
-// k = 8g+4+s. The order is fixed, so a tile's result is a deterministic
-// function of its inputs whatever worker computes it and however often it
-// is checkpointed and resumed.
+// k order: a k-step is two k-groups of 8; the lower half-wave supplies k =
+// 0-3 of both, the upper one k = 4-7. The order is fixed, so a tile's result
+// is a deterministic function of its inputs whatever worker computes it and
+// however often it is checkpointed and resumed.
 #pragma once
 #include "device.hpp"
 
 namespace apk {
 
-template <int G>
-struct EngMfma128T {
-  static_assert(G == 1 || G == 2, "stage groups of 1 or 2");
-  static constexpr int TM = 128, TN = 128, KS = 32, NS = G == 2 ? 4 : 3, GROUP = G,
-                       THREADS = 256;
-  // Pairs take tiles of an even number of k-stages only (a stage past the
-  // tile's end refetches the last one, which a pair would compute): the
-  // launches pick the one-stage ring for the others.
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+struct EngMfma128 {
+  static constexpr int TM = 128, TN = 128, KS = 32, NS = 3, GROUP = 1, THREADS = 256;
   // Waves per SIMD at most (1 block per CU (LDS-bound)): the register budget the
   // compiler may schedule for.
-  static constexpr int WAVES_PER_SIMD = 1;
+  static constexpr int WAVES_PER_SIMD = 1, BLOCKS_PER_CU = 1;
   static constexpr int MIN_WAVES_PER_SIMD = 1;  // occupancy the registers must allow
   static constexpr int A_STAGE = TM * KS * 4;               // bytes
   static constexpr int B_STAGE = KS * TN * 4;               // bytes
   static constexpr int STAGE = A_STAGE + B_STAGE;           // 32 KiB
-  static constexpr int LDS_BYTES = NS * STAGE;              // 96 / 128 KiB
+  // The split operands of two k-steps (planes), behind the ring.
+  static constexpr int BLOCK_PLANES = 3 * 64 * 16;          // one 32-row block: 3 KiB
+  static constexpr int PLANES = 8 * BLOCK_PLANES;           // a k-step's: 24 KiB
+  static constexpr int LDS_BYTES = NS * STAGE + 2 * PLANES; // 144 KiB
   static constexpr int LOADS_A = A_STAGE / (THREADS * 16);  // 4 per thread
   static constexpr int LOADS_B = B_STAGE / (THREADS * 16);  // 4 per thread
   static constexpr int LOADS = LOADS_A + LOADS_B;           // per stage
@@ -68,6 +85,7 @@ struct EngMfma128T {
 
   struct Acc {
     f32x16 c[2][2];
+    u16x2 tiny;  // smallest operands seen (tiny_watch)
   };
 
   static __device__ __forceinline__ int aswz(int r) { return (r ^ ((r >> 3) & 1)) & 7; }
@@ -95,6 +113,7 @@ struct EngMfma128T {
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) a.c[i][j][r] = 0.0f;
+    a.tiny = u16x2{0xffff, 0xffff};
   }
 
   // Direct-to-LDS loads of one k-stage. A load i (< 4) fills the 1 KiB
@@ -159,56 +178,250 @@ struct EngMfma128T {
 
   // Operands of k-group g (8 k values): one 16-byte A read per 32-row
   // block (the quad 2g+h of the lane's row), four B dwords per 32-column
-  // block.
+  // block (compute_exact). The wave's blocks are numbered so that block 0 of A is another
+  // one for its neighbour in the column, and block 0 of B for its neighbour
+  // in the row (arow, bcol): each wave watches its blocks 0 for small
+  // operands (tiny_watch), and together the four watch every operand once.
   struct Frag {
     f32x4 a4[2];
     float bv[2][4];
   };
+  static __device__ __forceinline__ int arow(int rb) {
+    const int w = threadIdx.x >> 6;
+    return (w & 1) * 64 + (rb ^ (w >> 1)) * 32;
+  }
+  static __device__ __forceinline__ int bcol(int cb) {
+    const int w = threadIdx.x >> 6;
+    return (w >> 1) * 64 + (cb ^ (w & 1)) * 32;
+  }
   static __device__ __forceinline__ void load_frag(const char* abase, int g, Frag& f) {
-    const int w = threadIdx.x >> 6, l = lane_id();
-    const int wm = w & 1, wn = w >> 1;
+    const int l = lane_id();
     const int lr = l & 31, h = l >> 5;
     const float* bbase = (const float*)(abase + A_STAGE);
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
-      const int row = wm * 64 + rb * 32 + lr;
+      const int row = arow(rb) + lr;
       const int q = (2 * g + h) ^ aswz(row);
       f.a4[rb] = *(const f32x4*)(abase + row * 128 + q * 16);
     }
     // Row k = 8g + 4h + s has bswz(k) = h << 3 for every s.
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb) {
-      const int col = wn * 64 + cb * 32 + lr;
+      const int col = bcol(cb) + lr;
       const int cpos = (((col >> 2) ^ (h << 3)) << 2) | (col & 3);
 #pragma unroll
       for (int s = 0; s < 4; ++s) f.bv[cb][s] = bbase[(8 * g + 4 * h + s) * TN + cpos];
     }
   }
 
-  // NST consecutive k-stages of MFMAs out of ring slots slot .. slot+NST-1
-  // (contiguous in LDS), as one sequence of k-groups in ascending k. The
-  // operands of group g+1 are read from LDS while group g's 16 MFMAs run.
-  // `pre` runs after the first group's operand reads are issued (the
-  // preempt-flag check: its LDS read overlaps theirs); if it returns false
-  // the stages are abandoned before any accumulator changes and the call
-  // returns false. `mid(i)`, i = 0..NST*LOADS-1, runs after MFMA 2i+1 of the
-  // first groups (8 per group): the stage loops issue the next stages'
-  // direct-to-LDS load i there, under the matrix work.
-  template <int NST, class Pre, class Mid>
-  static __device__ __forceinline__ bool compute_n(const char* ring, int slot, Acc& acc,
-                                                   Pre&& pre, Mid&& mid) {
+  // A k-step is two k-groups (16 k). Its operands are split: x = hi + mid +
+  // lo, each the round-to-nearest bf16 of what the former leave (24
+  // significand bits in all), eight k values of a row (column) per lane --
+  // the operand layout of v_mfma_f32_32x32x16_bf16, k in the order of the
+  // two groups. A wave splits its own blocks (A's block 0 and B's block 0)
+  // and takes the other two from the waves beside it, through LDS.
+  struct Own {
+    u32x4 a[3], b[3];  // 0 hi, 1 mid, 2 lo
+  };
+  struct Raw {
+    f32x4 a[2];
+    float b[8];
+  };
+  static constexpr int STEPS = KS / 16;       // k-steps per stage
+  static constexpr int MF = 24;               // MFMAs of a step per wave
+  static __device__ __forceinline__ void load_raw(const char* abase, int j, Raw& r) {
+    const int l = lane_id();
+    const int lr = l & 31, h = l >> 5;
+    const float* bbase = (const float*)(abase + A_STAGE);
+    const int row = arow(0) + lr, col = bcol(0) + lr;
+    const int cpos = (((col >> 2) ^ (h << 3)) << 2) | (col & 3);
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+      r.a[g] = *(const f32x4*)(abase + row * 128 + (((2 * (2 * j + g) + h) ^ aswz(row)) << 4));
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) r.b[4 * g + s] = bbase[(16 * j + 8 * g + 4 * h + s) * TN + cpos];
+  }
+  // Splits the wave's blocks in 24 parts, three for each of 8 value pairs
+  // (pairs 0-3 are A's, 4-7 B's): part 0 of a pair gives hi and what it
+  // leaves, part 1 mid, part 2 lo. One part goes under each MFMA: five vector
+  // instructions fit the 32 cycles of one, while more in a row, or two
+  // MFMAs in a row, leave one of the two units idle (a wave issues in
+  // order).
+  struct Rest {
+    float x0, x1;
+  };
+  static __device__ __forceinline__ void split_part(const Raw& r, int part, Own& d, Rest& rest,
+                                                    Acc& acc) {
+    const int p = part / 3, e = 2 * (p & 3);  // elements e, e + 1
+    u32x4* o = p < 4 ? d.a : d.b;
+    if (part % 3 == 0) {
+      const float x0 = p < 4 ? r.a[e >> 2][e & 3] : r.b[e];
+      const float x1 = p < 4 ? r.a[e >> 2][(e & 3) + 1] : r.b[e + 1];
+      const unsigned hi = pack(x0, x1);
+      rest = Rest{x0 - low(hi), x1 - high(hi)};
+      o[0][p & 3] = hi;
+    } else if (part % 3 == 1) {
+      const unsigned mid = pack(rest.x0, rest.x1);
+      rest = Rest{rest.x0 - low(mid), rest.x1 - high(mid)};
+      o[1][p & 3] = mid;
+    } else {
+      o[2][p & 3] = pack(rest.x0, rest.x1);
+      tiny_watch(o[0][p & 3], acc);
+    }
+  }
+  // This lane's 16 bytes of plane 0 of block `blk` (0-3 A's rows, 4-7 B's
+  // columns) of k-step buffer `buf`; planes 1 and 2 follow 1 KiB apart.
+  static __device__ __forceinline__ char* plane(char* ring, int buf, int blk) {
+    return ring + NS * STAGE + buf * PLANES + blk * BLOCK_PLANES + lane_id() * 16;
+  }
+  static __device__ __forceinline__ int ablock(int rb) { return arow(rb) >> 5; }
+  static __device__ __forceinline__ int bblock(int cb) { return 4 + (bcol(cb) >> 5); }
+  static __device__ __forceinline__ void put(char* dst, const u32x4 (&v)[3]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) *(u32x4*)(dst + i * 1024) = v[i];
+  }
+  static __device__ __forceinline__ void take(const char* src, u32x4 (&v)[3]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) v[i] = *(const u32x4*)(src + i * 1024);
+  }
+  // Two values rounded to bf16 (one v_cvt_pk_bf16_f32), and back.
+  static __device__ __forceinline__ unsigned pack(float x0, float x1) {
+    const f32x2 v = {x0, x1};
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+  }
+  static __device__ __forceinline__ float low(unsigned u) { return __uint_as_float(u << 16); }
+  static __device__ __forceinline__ float high(unsigned u) {
+    return __uint_as_float(u & 0xffff0000u);
+  }
+  // Keeps the smallest non-zero magnitude seen, as twice the bf16 bits less
+  // one (the sign falls out, and zero wraps to the largest value).
+  static __device__ __forceinline__ void tiny_watch(unsigned hi, Acc& acc) {
+    unsigned t;  // both halves: 2 x - 1
+    asm("v_pk_mad_u16 %0, %1, 2, -1 op_sel_hi:[1,0,1]" : "=v"(t) : "v"(hi));
+    acc.tiny = __builtin_elementwise_min(acc.tiny, __builtin_bit_cast(u16x2, t));
+  }
+  // MFMA m (< 24) of a k-step. Blocks in the order (own, own), (own, other),
+  // (other, own), (other, other), each with its six products in ascending
+  // size: mid.mid, lo.hi, hi.lo, mid.hi, hi.mid, hi.hi (the three left out
+  // are below 2^-24 of hi.hi). The wave's own come first: the others' planes
+  // arrive from LDS under them.
+  static __device__ __forceinline__ void mma(const Own& own, const Own& other, int m, Acc& acc) {
+    constexpr int PA[6] = {1, 2, 0, 1, 0, 0}, PB[6] = {1, 0, 2, 0, 1, 0};
+    const int t = m % 6, rb = m / 12, cb = m / 6 & 1;
+    const u32x4 a = (rb ? other : own).a[PA[t]], b = (cb ? other : own).b[PB[t]];
+    acc.c[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+        __builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc.c[rb][cb], 0, 0, 0);
+  }
+
+  // The k-steps are software-pipelined three deep, across the stage barriers:
+  // with one wave per SIMD nothing else covers an LDS round trip or a chain
+  // of conversions. A phase runs the MFMAs of one k-step while it splits the
+  // wave's own blocks of the next (read from the ring a phase earlier), puts
+  // them into the planes, and reads the blocks of the one after; a barrier
+  // later every wave takes the others' from the planes. What is left over
+  // from one call to the next: the own split blocks of a step whose MFMAs are
+  // to come (the others' lie in planes 0 by the next barrier) and the blocks
+  // of the step after it, not yet split.
+  struct Tail {
+    Own own;
+    Raw raw;
+  };
+  // The MFMAs of the step whose own blocks are `cur` (the others' in planes
+  // `buf`); under them `raw` is split into `next` and planes buf ^ 1 (SPLIT),
+  // and `mid(i)`, i = lo..lo+3, issues loads (four of them).
+  template <bool SPLIT, class Read, class Mid>
+  static __device__ __forceinline__ void phase(char* ring, int buf, const Own& cur,
+                                               const Raw& raw, Own& next, Acc& acc, Read&& read,
+                                               int lo, Mid&& mid) {
+    Own other;
+    Rest rest;
+    take(plane(ring, buf, bblock(1)), other.b);
+    take(plane(ring, buf, ablock(1)), other.a);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = 0; m < MF; ++m) {
+      mma(cur, other, m, acc);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (SPLIT) split_put(ring, buf ^ 1, raw, m, next, rest, acc);
+      if (m == 6) {
+        read();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (m % 5 == 4 && m / 5 < LOADS / 2) {
+        mid(lo + m / 5);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  // Part `part`; a block goes to the planes once its last part is done.
+  static __device__ __forceinline__ void split_put(char* ring, int buf, const Raw& raw, int part,
+                                                   Own& d, Rest& rest, Acc& acc) {
+    split_part(raw, part, d, rest, acc);
+    if (part == 11) put(plane(ring, buf, ablock(0)), d.a);
+    if (part == 23) put(plane(ring, buf, bblock(0)), d.b);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // Stage `slot` of the ring enters the pipeline; the two steps before it
+  // leave it (hasTail = false: there are none). `mid(i)`, i = 0..LOADS-1,
+  // issues the loads of a later stage, spread over the MFMAs.
+  template <class Mid>
+  static __device__ __forceinline__ void stage(char* ring, int slot, Acc& acc, Tail& t,
+                                               bool hasTail, Mid&& mid) {
+    static_assert(STEPS == 2 && LOADS == 8, "two phases per stage, four loads each");
     const char* abase = ring + slot * STAGE;
-    constexpr int GS = KS / 8;    // k-groups per stage
-    constexpr int GG = GS * NST;  // k-groups in all
+    Raw raw;
+    if (hasTail) {
+      Own odd;
+      phase<true>(ring, 0, t.own, t.raw, odd, acc, [&] { load_raw(abase, 0, raw); }, 0, mid);
+      lds_sync();
+      phase<true>(ring, 1, odd, raw, t.own, acc, [&] { load_raw(abase, 1, t.raw); }, 4, mid);
+    } else {
+      Rest rest;
+      load_raw(abase, 0, raw);
+      load_raw(abase, 1, t.raw);
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) mid(i);
+#pragma unroll
+      for (int p = 0; p < MF; ++p) split_put(ring, 0, raw, p, t.own, rest, acc);
+    }
+  }
+  // The two steps left over, before the accumulators are read.
+  static __device__ __forceinline__ void finish_tail(char* ring, Acc& acc, const Tail& t) {
+    Own odd;
+    lds_sync();  // every wave's planes
+    phase<true>(ring, 0, t.own, t.raw, odd, acc, [] {}, 0, [](int) {});
+    lds_sync();
+    phase<false>(ring, 1, odd, t.raw, odd, acc, [] {}, 0, [](int) {});
+  }
+
+  // Whether the tile must be computed again with exact products (this lane):
+  // a non-finite accumulator -- an operand or a sum was infinite, NaN or
+  // beyond bf16's largest value --, or an operand whose lowest bits bf16 may
+  // not hold (below 2^-100; lo's last bit of anything larger is a normal
+  // number).
+  static constexpr unsigned short TINY = 2 * ((127 - 100) << 7) - 1;
+  static __device__ __forceinline__ bool suspect(const Acc& a) {
+    float z[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) z[j] = fmaf(a.c[i][j][r], 0.0f, z[j]);
+    return !(z[0] + z[1] == 0.0f) || a.tiny[0] < TINY || a.tiny[1] < TINY;
+  }
+  // One k-stage with the exact fp32 products of v_mfma_f32_32x32x2_f32 (the
+  // path of tiles with suspect() operands).
+  static __device__ __forceinline__ void compute_exact(const char* ring, int slot, Acc& acc) {
+    const char* abase = ring + slot * STAGE;
+    constexpr int GG = KS / 8;
     Frag f[2];
     load_frag(abase, 0, f[0]);
-    if (!pre()) return false;
 #pragma unroll
     for (int g = 0; g < GG; ++g) {
-      // The reads of group g+1 are issued ahead of group g's 16 MFMAs (the
-      // scheduling barrier keeps the compiler from sinking each read next to
-      // its first use, where the LDS latency would stall the matrix pipe).
-      if (g + 1 < GG) load_frag(abase + ((g + 1) / GS) * STAGE, (g + 1) % GS, f[(g + 1) & 1]);
+      if (g + 1 < GG) load_frag(abase, g + 1, f[(g + 1) & 1]);
       __builtin_amdgcn_sched_barrier(0);
       const Frag& c = f[g & 1];
 #pragma unroll
@@ -216,36 +429,25 @@ struct EngMfma128T {
         const int s = m >> 2, rb = (m >> 1) & 1, cb = m & 1;
         acc.c[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(c.a4[rb][s], c.bv[cb][s],
                                                              acc.c[rb][cb], 0, 0, 0);
-        if ((m & 1) && g * 8 + (m >> 1) < NST * LOADS) {
-          __builtin_amdgcn_sched_barrier(0);
-          mid(g * 8 + (m >> 1));
-          __builtin_amdgcn_sched_barrier(0);
-        }
       }
     }
-    return true;
-  }
-  // The ring's stage group (GROUP stages).
-  template <class Pre, class Mid>
-  static __device__ __forceinline__ bool compute(const char* ring, int slot, Acc& acc,
-                                                 Pre&& pre, Mid&& mid) {
-    return compute_n<GROUP>(ring, slot, acc, static_cast<Pre&&>(pre), static_cast<Mid&&>(mid));
-  }
-  static __device__ __forceinline__ void compute(const char* ring, int slot, Acc& acc) {
-    compute(ring, slot, acc, [] { return true; }, [](int) {});
   }
 
   // Output element (tile-relative row, col) of accumulator register e.
   static __device__ __forceinline__ void coord(int e, int& r, int& c) {
-    const int w = threadIdx.x >> 6, l = lane_id();
-    const int wm = w & 1, wn = w >> 1, rb = e >> 5, cb = (e >> 4) & 1, q = e & 15;
-    r = wm * 64 + rb * 32 + 8 * (q >> 2) + 4 * (l >> 5) + (q & 3);
-    c = wn * 64 + cb * 32 + (l & 31);
+    const int l = lane_id();
+    const int rb = e >> 5, cb = (e >> 4) & 1, q = e & 15;
+    r = arow(rb) + 8 * (q >> 2) + 4 * (l >> 5) + (q & 3);
+    c = bcol(cb) + (l & 31);
   }
+  // A checkpoint carries `tiny` as a NaN in the lane's first accumulator: the
+  // resumed tile then ends suspect, as this one would have.
   static __device__ __forceinline__ float get(const Acc& a, int e) {
+    if (e == 0 && (a.tiny[0] < TINY || a.tiny[1] < TINY)) return __builtin_nanf("");
     return a.c[e >> 5][(e >> 4) & 1][e & 15];
   }
   static __device__ __forceinline__ void set(Acc& a, int e, float v) {
+    if (e == 0) a.tiny = u16x2{0xffff, 0xffff};
     a.c[e >> 5][(e >> 4) & 1][e & 15] = v;
   }
 
@@ -253,8 +455,7 @@ struct EngMfma128T {
   // is free once a tile's last stage has been computed).
   static __device__ __forceinline__ int pass_row(int, int rr) { return rr; }
   static __device__ __forceinline__ void stage_pass(const Acc& acc, char* lds, int) {
-    const int w = threadIdx.x >> 6, l = lane_id();
-    const int wm = w & 1, wn = w >> 1;
+    const int l = lane_id();
     const int lr = l & 31, h = l >> 5;
     float* t = (float*)lds;
 #pragma unroll
@@ -263,13 +464,10 @@ struct EngMfma128T {
       for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int row = wm * 64 + rb * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-          t[row * TN + wn * 64 + cb * 32 + lr] = acc.c[rb][cb][r];
+          const int row = arow(rb) + 8 * (r >> 2) + 4 * h + (r & 3);
+          t[row * TN + bcol(cb) + lr] = acc.c[rb][cb][r];
         }
   }
 };
-
-using EngMfma128 = EngMfma128T<1>;
-using EngMfma128Pairs = EngMfma128T<2>;
 
 }  // namespace apk

@@ -26,6 +26,7 @@ __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu
   __shared__ __attribute__((aligned(16))) char ring[E::LDS_BYTES];
   __shared__ unsigned s_task;
   __shared__ proto::QueueCursor s_cur;  // thread 0's place in the queue
+  __shared__ int s_suspect;
 
   const int tilesN = N / E::TN;
   const unsigned numTasks = (unsigned)((M / E::TM) * tilesN);
@@ -37,6 +38,7 @@ __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu
   const typename E::Ctx ctx = E::make_ctx(A, B, M, N, K);
   const uint32_t wl = wave_lds(ring);
   if (threadIdx.x == 0) {
+    s_suspect = 0;
     s_cur = proto::QueueCursor{0, 0, 0, 0, 0};
     tq.start(s_cur, blockIdx.x);
   }
@@ -62,7 +64,7 @@ __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu
     // one uniform compare per stage instead of a modulo under a per-thread
     // branch at the top of every stage.
     int nextRec = rec ? 0 : INT_MAX;
-    run_stages<E>(ring, wl, ctx, acc, row0, col0, K / E::KS, [&](int s) {
+    run_stages<E>(ring, wl, ctx, acc, row0, col0, K / E::KS, &s_suspect, [&](int s) {
       if (s != nextRec) return;
       nextRec += spc;
       if (threadIdx.x == 0) {
@@ -106,13 +108,15 @@ __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu
                    unsigned long long* end_gt) {
   if (start_gt && blockIdx.x == 0 && threadIdx.x == 0) *start_gt = (long long)wall_ticks();
   __shared__ __attribute__((aligned(16))) char ring[E::LDS_BYTES];
+  __shared__ int s_suspect;
+  if (threadIdx.x == 0) s_suspect = 0;  // first read after a stage's barrier
   const int tilesN = N / E::TN;
   const int row0 = (int)(blockIdx.x / (unsigned)tilesN) * E::TM;
   const int col0 = (int)(blockIdx.x % (unsigned)tilesN) * E::TN;
   const typename E::Ctx ctx = E::make_ctx(A, B, M, N, K);
   typename E::Acc acc;
   E::zero(acc);
-  run_stages<E>(ring, wave_lds(ring), ctx, acc, row0, col0, K / E::KS, [](int) {});
+  run_stages<E>(ring, wave_lds(ring), ctx, acc, row0, col0, K / E::KS, &s_suspect, [](int) {});
   store_tile<E>(acc, ring, C, N, row0, col0, false);
   if (end_gt) {
     wait_vmcnt<0>();  // this thread's C stores have completed
@@ -227,13 +231,6 @@ extern "C" int apk_persistent_gemm(int engine, const void* A, const void* B,
                                                next_task, log, blocks,
                                                as_stream(stream));
     case APK_ENGINE_MFMA128:
-      // Stage pairs (one barrier per 64 k) for tiles of whole pairs, except
-      // where per-chunk records are asked for at chunks that end inside a pair.
-      if (K % (2 * EngMfma128Pairs::KS) == 0 &&
-          (log == nullptr || k_chunk % (2 * EngMfma128Pairs::KS) == 0))
-        return launch_persistent_gemm<EngMfma128Pairs>(A, B, C, M, N, K, k_chunk,
-                                                       next_task, log, blocks,
-                                                       as_stream(stream));
       return launch_persistent_gemm<EngMfma128>(A, B, C, M, N, K, k_chunk,
                                                 next_task, log, blocks,
                                                 as_stream(stream));
@@ -259,16 +256,7 @@ extern "C" int apk_persistent_gemm_occupancy(int engine, int* blocks_per_cu) {
   using namespace apk;
   switch (engine) {
     case APK_ENGINE_VALU64: return occupancy_of<EngValu64>(blocks_per_cu);
-    case APK_ENGINE_MFMA128: {
-      // the smaller of the two ring shapes' occupancies (both 1 per CU)
-      int a = 0, b = 0;
-      const int rc = occupancy_of<EngMfma128>(&a);
-      if (rc != APK_OK) return rc;
-      const int rc2 = occupancy_of<EngMfma128Pairs>(&b);
-      if (rc2 != APK_OK) return rc2;
-      *blocks_per_cu = a < b ? a : b;
-      return APK_OK;
-    }
+    case APK_ENGINE_MFMA128: return occupancy_of<EngMfma128>(blocks_per_cu);
     case APK_ENGINE_BF16X256: return occupancy_of<EngBf16x256>(blocks_per_cu);
     case APK_ENGINE_BF16X128: return occupancy_of<EngBf16x128>(blocks_per_cu);
     case APK_ENGINE_BF16X256X128: return occupancy_of<EngBf16x256x128>(blocks_per_cu);
@@ -321,9 +309,6 @@ extern "C" int apk_urgent_gemm(int engine, const void* A, const void* B, float* 
     case APK_ENGINE_VALU64:
       return launch_urgent_tiles<EngValu64>(A, B, C, M, N, K, start_gt, end_gt, as_stream(stream));
     case APK_ENGINE_MFMA128:
-      if (K % (2 * EngMfma128Pairs::KS) == 0)
-        return launch_urgent_tiles<EngMfma128Pairs>(A, B, C, M, N, K, start_gt, end_gt,
-                                                    as_stream(stream));
       return launch_urgent_tiles<EngMfma128>(A, B, C, M, N, K, start_gt, end_gt, as_stream(stream));
     case APK_ENGINE_BF16X256:
       return launch_urgent_tiles<EngBf16x256>(A, B, C, M, N, K, start_gt, end_gt, as_stream(stream));

@@ -61,6 +61,7 @@ k_persistent_yield(const apk_yield_params) {
   __shared__ long long s_serve_t1;   // start of the current service's urgent work
   __shared__ int s_fsync;            // synchronous flag read (syncPoll)
   __shared__ proto::QueueCursor s_cur;  // thread 0's place in the work queue
+  __shared__ int s_suspect;          // a lane ended its tile suspect (note_suspect)
 
   const int tid = threadIdx.x, bid = blockIdx.x;
   // Values the stage loop does not need are recomputed from the parameters
@@ -134,7 +135,10 @@ k_persistent_yield(const apk_yield_params) {
   if (tid < APK_STATS_PER_BLOCK) s_stats[tid] = 0;
   if (tid < 3) s_setter[tid] = 0;
   if (tid < 2) s_due[tid] = 1;  // the first site sets the time base
-  if (tid == 0) s_cur = proto::QueueCursor{0, 0, 0, 0, 0};
+  if (tid == 0) {
+    s_cur = proto::QueueCursor{0, 0, 0, 0, 0};
+    s_suspect = 0;
+  }
   if (P().run_gt && bid == 0 && tid == 0) P().run_gt[0] = wall_ticks();
   __syncthreads();
   if constexpr (retreatArm) {
@@ -359,6 +363,9 @@ k_persistent_yield(const apk_yield_params) {
     bool hasTail = false;  // uniform
     // Not at issue sites, whose loop issues the next pair ahead of the poll.
     constexpr bool kPipe = PipelinedPairs<E>::value && POLL != APK_POLL_ISSUE;
+    // Single stages: the site check comes before the call, and a job that
+    // stops there runs its tail first.
+    constexpr bool kStagePipe = PipelinedStages<E>::value;
 
     // Poll sites are the stages s with s % pollStride == 0; `nextSite` is the
     // next one not yet passed (an urgent tile never reaches one), so a stage
@@ -542,12 +549,18 @@ k_persistent_yield(const apk_yield_params) {
           // s's matrix work; its slot held stage s-1, which every wave
           // finished before the barrier above.
           const typename E::Dst d = E::stage_dst(wl, ctx, aheadSlot, s + 2, S);
-          E::compute(ring, slot, acc, [] { return true; }, [&](int i) {
+          auto mid = [&](int i) {
             if constexpr (POLL != APK_POLL_ISSUE) {
               if (i == 0 && carry) sample(aheadSlot);
               E::issue_one(ctx, ln, d, i);
             }
-          });
+          };
+          if constexpr (kStagePipe) {
+            E::stage(ring, slot, acc, tail, hasTail, mid);
+            hasTail = true;
+          } else {
+            E::compute(ring, slot, acc, [] { return true; }, mid);
+          }
           slot = next_slot<E>(slot);
           ++s;
         } else {
@@ -623,6 +636,10 @@ k_persistent_yield(const apk_yield_params) {
           slot = other;
           s += 2;
         }
+      }
+      if constexpr (kStagePipe) {
+        if (hasTail) E::finish_tail(ring, acc, tail);
+        hasTail = false;
       }
       if (!atSite) break;  // the tile is computed
 
@@ -839,11 +856,16 @@ k_persistent_yield(const apk_yield_params) {
     if (retreated) break;  // the block exits; its tile waits in the resume queue
     if (yielded) continue;  // the event's urgent tiles first, then this tile again
     if constexpr (kPipe) {
-      if (hasTail) E::finish_tail(acc, tail);
+      if (hasTail) E::finish_tail(ring, acc, tail);
     }
+    note_suspect<E>(acc, &s_suspect);
     wait_vmcnt<0>();  // the refetches past the tile's end have landed
     lds_sync();       // every wave done with the ring; every sample has landed
     if (POLL != APK_POLL_OFF && lastSlot >= 0) fLatest = uniform(flagring[lastSlot]);
+    // (The poison control's staged operands are gone by now, and its tiles
+    // are wrong on purpose.)
+    if (take_suspect<E>(&s_suspect) && !(urgent && P().poison))
+      run_exact<E>(ring, wl, ctx, acc, row0, col0, S);
 
     // ---- epilogue: C tile, fingerprint, exactly-once count ----
     float* C = urgent ? P().Cu + (size_t)serving * (size_t)P().cu_event_stride : P().C;

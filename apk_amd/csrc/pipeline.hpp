@@ -160,7 +160,24 @@ struct PipelinedPairs {
 };
 template <class E>
 struct PipelinedPairs<E, true> {
-  static constexpr bool value = E::BLOCKS_PER_CU == 1;
+  static constexpr bool value = E::GROUP == 2 && E::BLOCKS_PER_CU == 1;
+};
+// The same for the ring of single stages: an engine with a tail defers it
+// there whatever the kernel.
+template <class E>
+struct PipelinedStages {
+  static constexpr bool value = E::GROUP == 1 && HasTailPipe<E>::value;
+};
+// An engine that computes with split operands (E::suspect, E::compute_exact):
+// a tile one of whose lanes ends suspect is computed again with exact
+// products.
+template <class E, class = void>
+struct HasExact {
+  static constexpr bool value = false;
+};
+template <class E>
+struct HasExact<E, std::void_t<decltype(&E::suspect)>> {
+  static constexpr bool value = true;
 };
 template <class E>
 __device__ __forceinline__ void issue_group_one(const typename E::Ctx& c,
@@ -175,19 +192,63 @@ __device__ __forceinline__ void issue_group_one(const typename E::Ctx& c,
   }
 }
 
+// The exact products of a tile whose operands are suspect: rare, so a plain
+// loop over two ring slots that keeps no state of the caller's loop. Every
+// wave has finished with the ring when it is called and when it returns.
+template <class E>
+__device__ __forceinline__ void run_exact(char* ring, uint32_t wl, const typename E::Ctx& c,
+                                          typename E::Acc& acc, int row0, int col0, int S) {
+  if constexpr (HasExact<E>::value) {
+    const typename E::Lane ln = E::lane_offsets(c, row0, col0);
+    E::zero(acc);
+    issue_loads<E>(c, ln, E::stage_dst(wl, c, 0, 0, S));
+#pragma unroll 1
+    for (int s = 0; s < S; ++s) {
+      issue_loads<E>(c, ln, E::stage_dst(wl, c, (s + 1) & 1, s + 1, S));
+      wait_vmcnt<E::LOADS>();
+      lds_sync();
+      E::compute_exact(ring, s & 1, acc);
+      lds_sync();
+    }
+    wait_vmcnt<0>();
+    lds_sync();
+  }
+}
+// Whether any lane of the block ended its tile suspect: each wave notes it
+// in *flag (LDS, zero) before the barrier that ends the tile, and the block
+// reads it after (take_suspect, uniform; leaves *flag zero).
+template <class E>
+__device__ __forceinline__ void note_suspect(const typename E::Acc& acc, int* flag) {
+  if constexpr (HasExact<E>::value) {
+    if (E::suspect(acc)) *flag = 1;
+  }
+}
+template <class E>
+__device__ __forceinline__ bool take_suspect(int* flag) {
+  if constexpr (HasExact<E>::value) {
+    if (uniform(*flag) == 0) return false;
+    lds_sync();
+    if (threadIdx.x == 0) *flag = 0;
+    lds_sync();
+    return true;
+  }
+  return false;
+}
+
 // Non-preemptible K loop over stages [0, S) of one tile. hook(s) runs
-// uniformly before stage s is computed.
+// uniformly before stage s is computed. `flag`: a zeroed LDS word (see
+// note_suspect).
 template <class E, class Hook>
 __device__ __forceinline__ void run_stages(char* ring, uint32_t wl, const typename E::Ctx& c,
                                            typename E::Acc& acc, int row0, int col0, int S,
-                                           Hook&& hook) {
+                                           int* flag, Hook&& hook) {
   const typename E::Lane ln = E::lane_offsets(c, row0, col0);
   issue_loads<E>(c, ln, E::stage_dst(wl, c, 0, 0, S));
   issue_loads<E>(c, ln, E::stage_dst(wl, c, 1, 1, S));
   int slot = 0;
   // Pairs pipelined across the barrier (E::compute_pl), as in the
   // preemptible kernel with polls off.
-  constexpr bool kPipe = PipelinedPairs<E>::value;
+  constexpr bool kPipe = PipelinedPairs<E>::value || PipelinedStages<E>::value;
   typename TailFrag<E>::type tail;
   bool hasTail = false;
   for (int s = 0; s < S; s += E::GROUP) {
@@ -196,8 +257,13 @@ __device__ __forceinline__ void run_stages(char* ring, uint32_t wl, const typena
       wait_landed<E>();
       lds_sync();
       const typename E::Dst d = E::stage_dst(wl, c, slot_after_next(slot), s + 2, S);
-      E::compute(ring, slot, acc, [] { return true; },
-                 [&](int i) { E::issue_one(c, ln, d, i); });
+      auto mid = [&](int i) { E::issue_one(c, ln, d, i); };
+      if constexpr (kPipe) {
+        E::stage(ring, slot, acc, tail, hasTail, mid);
+        hasTail = true;
+      } else {
+        E::compute(ring, slot, acc, [] { return true; }, mid);
+      }
       slot = next_slot<E>(slot);
     } else {
       // The next pair's load descriptors are formed and pinned before the
@@ -222,10 +288,12 @@ __device__ __forceinline__ void run_stages(char* ring, uint32_t wl, const typena
     }
   }
   if constexpr (kPipe) {
-    if (hasTail) E::finish_tail(acc, tail);
+    if (hasTail) E::finish_tail(ring, acc, tail);
   }
+  note_suspect<E>(acc, flag);
   wait_vmcnt<0>();
   lds_sync();
+  if (take_suspect<E>(flag)) run_exact<E>(ring, wl, c, acc, row0, col0, S);
 }
 
 // ---------------------------------------------------------------------------

@@ -30,8 +30,13 @@ enum {
  *  VALU64   : 64x64 fp32 tile, 256 threads, one fmaf chain per output in the
  *             reference's k order (src/tile.cuh:62-107) -- bit-identical to a
  *             correctly rounded sequential fmaf over k.
- *  MFMA128  : 128x128 fp32 tile on v_mfma_f32_32x32x2_f32 (fp32 matrix
- *             cores), 256 threads, 3-stage LDS ring fed by buffer_load ... lds.
+ *  MFMA128  : 128x128 fp32 tile on the matrix cores, 256 threads, 3-stage LDS
+ *             ring fed by buffer_load ... lds. Operands are split exactly into
+ *             three bf16 parts and multiplied by v_mfma_f32_32x32x16_bf16 with
+ *             fp32 accumulation (error against 64 bits below the fp32 chain's);
+ *             tiles with operands or sums that bf16's range cannot carry
+ *             (infinite, NaN, above 3.39e38, below 2^-100) are computed with
+ *             v_mfma_f32_32x32x2_f32 products.
  *  BF16X256 : 256x256 tile of a bf16 GEMM with fp32 accumulation on
  *             v_mfma_f32_32x32x16_bf16, 512 threads (two waves per SIMD),
  *             1 block per CU (replaces the reference's fp16 wmma tile,

@@ -1,0 +1,114 @@
+"""The fp32 MFMA tile's split products (three bf16 parts per operand) on the
+GPU: no less exact than the fp32 chain over the range of K, and operands that
+the parts cannot carry (infinite, NaN, above bf16's range, below 2^-100)
+computed with exact products, also through checkpoint and resume.
+
+Bound for finite results: each C element sums K products in fp32, at most K
+roundings of 2^-24 each, and three products of parts below 2^-24 of a b are
+left out, so |C - C64| <= (K + 4) 2^-24 (|A| |B|) + (K + 1) 2^-149 (the last
+term where sums are denormal)."""
+import numpy as np
+import pytest
+
+import oracle
+from gpu_util import run_persistent, say
+from test_gpu_yield import Job, _bits, _blocks
+
+pytestmark = pytest.mark.gpu
+
+
+def _bound(A, B):
+    K = A.shape[1]
+    mag = np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64)
+    return (K + 4) * 2.0 ** -24 * mag + (K + 1) * 2.0 ** -149
+
+
+@pytest.mark.parametrize("K", [32, 64, 96, 128, 992])
+def test_split_no_less_exact_than_the_chain(torch_gpu, apk, K):
+    """One stage (pipeline filled and drained at once), two, an odd number, many."""
+    say(f"mfma128 split error, M=256 N=384 K={K}")
+    A, B = oracle.fill_uniform_pm1(17, 256, 384, K)
+    C, _, _ = run_persistent(torch_gpu, apk, apk.ENGINE_MFMA128, A, B, K, blocks=5, with_log=False)
+    ref = oracle.gemm_f64(A, B, threads=8)
+    chain = oracle.gemm_f32_chain(A, B)
+    err, err_chain = oracle.rel_frobenius(C, ref), oracle.rel_frobenius(chain, ref)
+    say(f"  rel-Frobenius {err:.2e}, fp32 chain {err_chain:.2e}")
+    assert (np.abs(C - ref) <= _bound(A, B)).all()
+    assert err <= 1.1 * err_chain  # two independent samples of rounding noise
+
+
+def _special(kind):
+    A, B = oracle.fill_uniform_pm1(5, 256, 256, 96)
+    if kind == "tiny":        # all of A: lowest parts would be denormal or lost
+        A *= np.float32(2.0 ** -118)
+        B *= np.float32(2.0 ** 60)
+    elif kind == "tiny_one":  # one element of one row
+        A[200, 70] = np.float32(1.2345678 * 2.0 ** -120)
+        A[200, :70] = A[200, 71:] = 0
+    elif kind == "denormal":
+        A[:, 5] = np.float32(2.0 ** -140)
+        B[5, :] *= np.float32(2.0 ** 100)
+    elif kind == "huge":      # above bf16's largest value, finite products
+        A[7, 3] = np.float32(3.4028e38)
+        B[3, :] *= np.float32(2.0 ** -20)
+    elif kind == "inf":
+        A[130, 95] = np.inf
+    elif kind == "inf_zero":  # inf * 0 = NaN, in one row only
+        A[1, 2] = np.inf
+        B[2, 9] = 0
+    elif kind == "nan":
+        B[31, 200] = np.nan
+    elif kind == "overflow":  # finite operands, infinite sums
+        A[64] = np.float32(2.0 ** 100)
+        B[:, 64] = np.float32(2.0 ** 100)
+    elif kind == "zeros":     # signed zeros are ordinary operands
+        A[:, ::2] = -0.0
+        B[1::3] = 0.0
+    return A, B
+
+
+KINDS = ["tiny", "tiny_one", "denormal", "huge", "inf", "inf_zero", "nan", "overflow", "zeros"]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_split_special_operands(torch_gpu, apk, kind):
+    say(f"mfma128 special operands: {kind}")
+    A, B = _special(kind)
+    C, _, _ = run_persistent(torch_gpu, apk, apk.ENGINE_MFMA128, A, B, 96, blocks=3,
+                             with_log=False)
+    with np.errstate(all="ignore"):
+        chain = oracle.gemm_f32_chain(A, B)
+        finite = np.isfinite(chain)
+        assert np.array_equal(np.isnan(C), np.isnan(chain))
+        assert np.array_equal(C[~finite & ~np.isnan(chain)], chain[~finite & ~np.isnan(chain)])
+        ref = A.astype(np.float64) @ B.astype(np.float64)
+        A0, B0 = np.nan_to_num(A, posinf=0.0), np.nan_to_num(B)
+        bound = _bound(A0, B0)
+        assert (np.abs(C - ref)[finite] <= bound[finite]).all()
+
+
+@pytest.mark.parametrize("kind", ["tiny_one", "inf", "zeros"])
+@pytest.mark.parametrize("resume", [0, 1])
+def test_split_special_operands_through_yields(torch_gpu, apk, kind, resume):
+    """The small operand lies in the first stages of a tile that is then
+    checkpointed: the resumed tile must still be computed exactly."""
+    say(f"mfma128 special operands through yields: {kind} resume={resume}")
+    E = apk.ENGINE_MFMA128
+    j = Job(torch_gpu, apk, E, 256, 256, 1024, 32, 128, 128, 64, events=30,
+            blocks=min(8, _blocks(apk, E, apk.POLL_STAGE)), passes=20)
+    if kind == "tiny_one":
+        j.A[:, 8:] = 0
+        j.A[:, :8] *= np.float32(2.0 ** -120)
+    elif kind == "inf":
+        j.A[200, 3] = np.inf
+    else:
+        j.A[:, ::3] = -0.0
+    j.dA.copy_(torch_gpu.from_numpy(j.A))
+    off = j.run(apk.POLL_OFF, events=0)
+    r = j.run(apk.POLL_STAGE, resume=resume, gap_ticks=1000)
+    assert int(r["stats"][:, apk.ST_YIELDS].sum()) >= 5
+    assert (_bits(r["C"]) == _bits(off["C"])).all()
+    assert (r["task_hash"] == off["task_hash"]).all()
+    if kind == "tiny_one":
+        ref = j.A.astype(np.float64) @ j.B.astype(np.float64)
+        assert (np.abs(off["C"] - ref) <= _bound(j.A[:, :8], j.B[:8])).all()
