@@ -395,6 +395,16 @@ k_persistent_yield(const apk_yield_params) {
     // were issued nanoseconds earlier. `ahead`: that issue is already done
     // for the current s (re-entry after a site, or a restored ring).
     bool ahead = false;
+    // Single stages: stage s+2 (and the sample for the site at s+1), into the
+    // slot of stage s-1, which every wave finished before the barrier. A job
+    // with a tail polls first: a site that stops it runs the tail, some 3500
+    // cycles in which the loads would land, and then issues them, right
+    // before the checkpoint.
+    auto issue_ahead = [&] {
+      const int a = slot_after_next(slot);
+      if (pollable) sample(a);
+      issue_loads<E>(ctx, ln, E::stage_dst(wl, ctx, a, s + 2, S));
+    };
     // Stages resident or in flight, not yet computed, at a site before stage
     // st: what a FULL checkpoint keeps. With pairs the zero stage after an
     // odd tile's last stage is kept too (the pair is computed as a whole).
@@ -512,14 +522,8 @@ k_persistent_yield(const apk_yield_params) {
         // `pre` hook (measured: 10.8% -> 7-9% every-site overhead for the
         // bf16 engine, while the same placement cost the fp32 engines 1-2%).
         if constexpr (E::GROUP == 1) {
-          if constexpr (POLL == APK_POLL_ISSUE) {
-            // Stage s+2 (and the sample for the site at s+1) at once, into the
-            // slot of stage s-1, which every wave finished before the barrier.
-            if (!ahead) {
-              const int a = slot_after_next(slot);
-              if (pollable) sample(a);
-              issue_loads<E>(ctx, ln, E::stage_dst(wl, ctx, a, s + 2, S));
-            }
+          if constexpr (POLL == APK_POLL_ISSUE && !kStagePipe) {
+            if (!ahead) issue_ahead();
             ahead = false;
           }
           if (POLL != APK_POLL_OFF && s == nextSite) {
@@ -537,11 +541,15 @@ k_persistent_yield(const apk_yield_params) {
               if ((int)setter_due() | (f != lastSeen)) {
                 fSeen = f;
                 atSite = true;
-                ahead = POLL == APK_POLL_ISSUE;
+                if constexpr (!kStagePipe) ahead = POLL == APK_POLL_ISSUE;
                 break;
               }
             }
             nextSite += siteStride;
+          }
+          if constexpr (POLL == APK_POLL_ISSUE && kStagePipe) {
+            if (!ahead) issue_ahead();
+            ahead = false;
           }
           const int aheadSlot = slot_after_next(slot);
           const bool carry = s + 1 == nextSite;  // s+1 is a site
@@ -640,6 +648,10 @@ k_persistent_yield(const apk_yield_params) {
       if constexpr (kStagePipe) {
         if (hasTail) E::finish_tail(ring, acc, tail);
         hasTail = false;
+        if constexpr (POLL == APK_POLL_ISSUE) {
+          if (atSite && !ahead) issue_ahead();
+          ahead = atSite;
+        }
       }
       if (!atSite) break;  // the tile is computed
 
