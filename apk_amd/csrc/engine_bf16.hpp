@@ -475,5 +475,9 @@ using EngBf16x256 = EngBf16T<256, 256, 512, 1, 32, 1>;
 using EngBf16x128 = EngBf16T<128, 128, 64, 4, 16, 1>;
 // 256x128 on four waves, 2 blocks per CU: 16-deep stages, 32-k regions
 using EngBf16x256x128 = EngBf16T<256, 128, 256, 2, 16, 2>;
+// 128x128 on four waves (2x2, each 64x64), for urgent jobs of few tiles: the
+// same k order and K multiple as the tile it stands in for
+using EngBf16Urgent256 = EngBf16T<128, 128, 256, 2, 32, 1>;
+using EngBf16Urgent256x128 = EngBf16T<128, 128, 256, 2, 16, 1>;
 
 }  // namespace apk

@@ -195,15 +195,52 @@ static int scratch_of_current_device(unsigned** out) {
   return APK_OK;
 }
 
+// The tile an urgent job of few tiles is computed with: the latency of such a
+// job is that of one block's tile, so the bf16 tiles of several 128x128 parts
+// are handed to as many blocks instead (each tile's C is bit-identical, as
+// every output's sum has the same order): bf16x256 256^3 8.9 -> 4.1 us,
+// 512^3 13.2 -> 5.7, 1024x1024x4096 75 -> 42; bf16x256x128 512^3 8.7 -> 6.4,
+// 1024x1024x4096 71 -> 50. What bounds it: one wave per SIMD, whose operand
+// reads and MFMAs of a k-step follow the barrier of its load region.
+// The line: at most two such blocks per dispatch domain, which is what one CU
+// holds of them. An urgent job that waits for the retreat arm's freed CUs, one
+// per domain, then still starts at once; larger jobs keep the engine's own
+// tile.
+// The one-wave 128x128 tile stays as it is: a block that retreats beside it
+// frees the registers of one SIMD, and four waves may not fit there.
+constexpr int kUrgentParts = 2 * APK_RETREAT_DOMAINS;
+template <class E>
+struct UrgentTile {
+  using type = E;
+};
+template <>
+struct UrgentTile<EngBf16x256> {
+  using type = EngBf16Urgent256;
+};
+template <>
+struct UrgentTile<EngBf16x256x128> {
+  using type = EngBf16Urgent256x128;
+};
+
 template <class E>
 static int launch_urgent_tiles(const void* A, const void* B, float* C, int M, int N, int K,
                                long long* start_gt, unsigned long long* end_gt,
                                hipStream_t st) {
   const int rc = validate_persistent_gemm<E>(A, B, C, M, N, K, K, 1);
   if (rc != APK_OK) return rc;
-  const int tiles = (M / E::TM) * (N / E::TN);
-  hipLaunchKernelGGL(k_urgent_tiles<E>, dim3(tiles), dim3(E::THREADS), 0, st, A, B, C, M, N, K,
-                     start_gt, end_gt);
+  using U = typename UrgentTile<E>::type;
+  static_assert(E::TM % U::TM == 0 && E::TN % U::TN == 0 &&
+                    KAlign<E>::value == KAlign<U>::value && E::KS == U::KS,
+                "every shape that E takes is one of U's");
+  const long long parts = (long long)(M / U::TM) * (N / U::TN);
+  if (parts <= kUrgentParts) {
+    hipLaunchKernelGGL(k_urgent_tiles<U>, dim3((int)parts), dim3(U::THREADS), 0, st, A, B, C, M,
+                       N, K, start_gt, end_gt);
+  } else {
+    const int tiles = (M / E::TM) * (N / E::TN);
+    hipLaunchKernelGGL(k_urgent_tiles<E>, dim3(tiles), dim3(E::THREADS), 0, st, A, B, C, M, N, K,
+                       start_gt, end_gt);
+  }
   APK_LAUNCHED();
   return APK_OK;
 }

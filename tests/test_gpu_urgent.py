@@ -63,6 +63,38 @@ def test_urgent_bf16_matches_persistent(torch_gpu, apk, name):
     assert 0 < start <= end
 
 
+# Jobs of at most 64 128x128 parts are computed part by part: the smallest
+# (one part row, the least K), odd numbers of load regions, the last size on
+# the parts and the first on the engine's own tile.
+@pytest.mark.parametrize("name,M,N,K", [
+    ("bf16x256", 256, 256, 64), ("bf16x256", 256, 768, 192), ("bf16x256", 2048, 512, 128),
+    ("bf16x256", 2304, 512, 128), ("bf16x256x128", 256, 128, 32),
+    ("bf16x256x128", 512, 384, 160), ("bf16x256x128", 1024, 1024, 96),
+    ("bf16x256x128", 256, 4224, 96)])
+def test_urgent_bf16_parts(torch_gpu, apk, name, M, N, K):
+    torch = torch_gpu
+    eng = apk.ENGINES[name]
+    say(f"urgent_gemm {name} {M}x{N}x{K}: parts vs persistent_gemm")
+    gen = torch.Generator().manual_seed(M + N + K)
+    A = torch.randn(M, K, generator=gen).to(torch.bfloat16)
+    Bt = torch.randn(N, K, generator=gen).to(torch.bfloat16)
+    C, start, end = run_urgent(torch, apk, eng, A.view(torch.int16).numpy(),
+                               Bt.view(torch.int16).numpy())
+    dA, dB = A.cuda(), Bt.cuda()
+    dC = torch.full((M, N), float("nan"), device="cuda")
+    q = torch.zeros(apk.QUEUE_WORDS, dtype=torch.int32, device="cuda")
+    apk.persistent_gemm(eng, dA.data_ptr(), dB.data_ptr(), dC.data_ptr(), M, N, K, K,
+                        q.data_ptr(), None, 64, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    # the same products in the same order: not one bit may differ
+    assert np.array_equal(C.view(np.uint32), dC.cpu().numpy().view(np.uint32))
+    ref = oracle.gemm_f64(A.float().numpy(), np.ascontiguousarray(Bt.float().numpy().T), threads=8)
+    # exact products; at most K roundings of 2^-24 of a partial sum, whose rms is at
+    # most the result's
+    assert oracle.rel_frobenius(C, ref) <= 2.0 ** -24 * K
+    assert 0 < start <= end
+
+
 def test_urgent_rejects_bad_shape(torch_gpu, apk):
     # M = 100 is not a multiple of the 128-row tile: refused before any launch
     buf = torch_gpu.zeros(128 * 128, dtype=torch_gpu.float32, device="cuda")
