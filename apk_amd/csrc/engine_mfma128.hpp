@@ -451,6 +451,24 @@ struct EngMfma128 {
     a.c[e >> 5][(e >> 4) & 1][e & 15] = v;
   }
 
+  // The C tile straight from the accumulators: a register holds, in each
+  // half-wave, 32 consecutive columns of one row, so one dword store writes
+  // two whole 128-byte row segments, with no LDS and no barrier:
+  // 256^3 urgent 14.7 -> 14.0 us, 4096^3 804 -> 778.
+  // (A fingerprinted tile is staged in LDS instead.)
+  static __device__ __forceinline__ void store_direct(const Acc& acc, float* C, int ldc,
+                                                      int row0, int col0) {
+    const int l = lane_id();
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb) {
+        float* base = C + (size_t)(row0 + arow(rb) + 4 * (l >> 5)) * ldc + col0 + bcol(cb) + (l & 31);
+#pragma unroll
+        for (int q = 0; q < 16; ++q) base[(size_t)(8 * (q >> 2) + (q & 3)) * ldc] = acc.c[rb][cb][q];
+      }
+  }
+
   // Write the accumulators into LDS as the row-major TM x TN tile (the ring
   // is free once a tile's last stage has been computed).
   static __device__ __forceinline__ int pass_row(int, int rr) { return rr; }
