@@ -185,6 +185,7 @@ int apk_persistent_gemm_noalloc(int engine, const void* A, const void* B, float*
  * are resident in LDS and not yet computed (the "live" stages).
  *   APK_RESUME_CKPT_FULL : accumulators + the live LDS stages -> HBM -> back
  *   APK_RESUME_CKPT_ACC  : accumulators -> HBM -> back; live stages re-fetched
+ *                          (MFMA128: from one stage earlier, computed again)
  *   APK_RESUME_RESTART   : abandon the tile, restart it from k = 0 (the
  *                          reference's semantics, src/midyield.cu:237-258)
  * All three produce bit-identical C: the per-tile k order never changes.

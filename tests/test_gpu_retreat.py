@@ -218,6 +218,12 @@ def test_retreat_bit_identical_exactly_once(fp32_job, apk, poll, resume, pe):
     assert (_bits(r["Cu"]) == _bits(fp32_job.uref)).all(), "urgent output differs"
 
 
+# Accumulator checkpoints taken one stage before a chunk site.
+@pytest.mark.parametrize("pe", [1, 2])
+def test_retreat_chunk_accumulator_checkpoint(fp32_job, apk, pe):
+    _check(fp32_job, fp32_job.ref, fp32_job.run(1, apk.RESUME_CKPT_ACC, poll_every=pe))
+
+
 def test_retreat_bf16(torch_gpu, apk):
     say("building bf16x256 retreat job M=N=1024 K=2048 kc=256")
     job = RetreatJob(torch_gpu, apk, apk.ENGINE_BF16X256, 1024, 1024, 2048, 256, 256, 256, 256,

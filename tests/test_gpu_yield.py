@@ -175,6 +175,18 @@ def test_mfma128_yield_bit_identical(torch_gpu, apk, mfma_job, poll, resume):
     say(f"  fired {fired} events, {int(r['stats'][:, 0].sum())} yields, bit-identical")
 
 
+# An accumulator checkpoint is taken one stage before the site and resumed
+# there: chunk sites, every one and every second, counted across that stage.
+@pytest.mark.parametrize("poll_every", [1, 2])
+def test_mfma128_chunk_accumulator_checkpoint(torch_gpu, apk, mfma_job, poll_every):
+    say(f"mfma128 yield poll=chunk resume=acc poll_every={poll_every}")
+    j = mfma_job
+    off = j.run(apk.POLL_OFF, events=0)
+    _, u_ref_h = j.urgent_reference()
+    r = j.run(apk.POLL_CHUNK, resume=apk.RESUME_CKPT_ACC, poll_every=poll_every)
+    _assert_run_exact(j, r, off["C"], j.tile_hashes(off["C"]), u_ref_h)
+
+
 def test_mfma128_poison_is_detected(torch_gpu, apk, mfma_job):
     say("mfma128 poison control")
     j = mfma_job
