@@ -57,7 +57,7 @@ k_persistent_yield(const apk_yield_params) {
   // setter's state live in LDS: they are touched only off the stage loop.
   __shared__ unsigned long long s_stats[APK_STATS_PER_BLOCK];
   __shared__ long long s_setter[3];  // next event, time base, when it is due
-  __shared__ int s_due[2];           // due, as of the setter's last site / this one
+  __shared__ int s_due[2];           // the setter's look at the clock (SetterLook)
   __shared__ long long s_serve_t1;   // start of the current service's urgent work
   __shared__ int s_fsync;            // synchronous flag read (syncPoll)
   __shared__ proto::QueueCursor s_cur;  // thread 0's place in the work queue
@@ -185,17 +185,10 @@ k_persistent_yield(const apk_yield_params) {
   };
 
   // Whether the setter has something to do at this site (uniform; called
-  // once per site, after a barrier): thread 0 looked at the clock at the last
-  // one, and looks again now for the next. The block leaves the stage loop
-  // only then, not at every site: leaving drains the software pipeline, which
-  // would make the setter's tiles the slowest of the grid.
-  int dueSite = 0;  // uniform
+  // once per site, after a barrier).
+  proto::SetterLook<DevPlat> look{s_due, 0};
   auto setter_due = [&]() -> bool {
-    if (!isSetter) return false;
-    const bool due = uniform(s_due[dueSite]) != 0;
-    dueSite ^= 1;
-    if (tid == 0) s_due[dueSite] = wall_ticks() >= s_setter[2];
-    return due;
+    return isSetter && look.at_site(tid == 0, [&] { return wall_ticks() >= s_setter[2]; });
   };
 
   // Broadcast a value thread 0 computed (uniform afterwards).
@@ -690,7 +683,7 @@ k_persistent_yield(const apk_yield_params) {
         const long long at = ev < P().num_events ? gBase + P().sched[ev]
                              : P().stop_after > 0 ? stopAt : LLONG_MAX;
         s_setter[2] = at;
-        s_due[0] = s_due[1] = now >= at;
+        look.next(now >= at);
       }
       if (f > P().num_events) f = P().num_events;  // never index past the event arrays
       srcKind = AS_IS;

@@ -39,6 +39,7 @@ struct DevPlat {
   }
   static __device__ __forceinline__ int64_t ticks() { return wall_ticks(); }
   static __device__ __forceinline__ void pause() { __builtin_amdgcn_s_sleep(8); }
+  static __device__ __forceinline__ int uniform(int v) { return apk::uniform(v); }
 };
 
 using TaskQueue = proto::TaskQueue<DevPlat>;

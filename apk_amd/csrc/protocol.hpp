@@ -308,5 +308,33 @@ APK_PROTO_FN int retreat_role(bool continuation, int launch_epoch, int f) {
   return RETREAT_BY_QUOTA;
 }
 
+// ---------------------------------------------------------------------------
+// The setter block's look at the clock. At every poll site, right after the
+// site's barrier, each wave asks whether the setter has something to do
+// (at_site), and the block leaves its stage loop where it has: leaving drains
+// the software pipeline, which at every site would make the setter's tiles the
+// slowest of the grid. The answer must be the same for every wave, so it is
+// read from block memory: thread 0 looked at the clock at the last site, and
+// looks again now for the next. Two words, used in turn: the one a wave may
+// still be reading at this site is not written before the next site's
+// barrier -- neither by at_site nor, where the block has left the loop with
+// no barrier in between, by next().
+template <class P>
+struct SetterLook {
+  int* due;  // [2], block memory
+  int turn;  // uniform: the word that the next site reads
+
+  // Every thread, once per site. `look()` runs in thread 0 only.
+  template <class Look>
+  APK_PROTO_FN bool at_site(bool leader, Look&& look) {
+    const bool now = P::uniform(due[turn]) != 0;
+    turn ^= 1;
+    if (leader) due[turn] = look();
+    return now;
+  }
+  // Thread 0, between two sites: what the next one reads.
+  APK_PROTO_FN void next(bool v) const { due[turn] = v; }
+};
+
 }  // namespace proto
 }  // namespace apk

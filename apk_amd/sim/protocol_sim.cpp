@@ -40,6 +40,13 @@
 //                   first and decline when its entry stays taken past the
 //                   deadline (this leaves a hole in the ticket order)
 //   double-serve    (coop) serve the urgent tile popped by the previous block again
+//   due-both        (setter) write both words of the setter's look at a site
+//
+// --arm setter: the waves of the setter block alone (--waves of them), which
+// must agree at every poll site whether to leave the stage loop. Between two
+// barriers the waves run one after the other, in every order over the sites
+// (a barrier is all that orders them on the GPU); a block whose waves
+// disagree once is split over its barriers.
 //
 // Exit status 0 when every check passes, 1 otherwise; one summary line.
 #include <stdint.h>
@@ -47,6 +54,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <random>
@@ -90,6 +98,7 @@ struct HostPlat {
                std::chrono::steady_clock::now().time_since_epoch()).count() / 10;
   }
   static void pause() { std::this_thread::yield(); }
+  static int uniform(int v) { return v; }
 };
 namespace proto = apk::proto;
 
@@ -123,7 +132,8 @@ uint64_t expected(unsigned tile, int S, bool urgent) {
 }
 
 enum Resume { R_FULL = 2, R_ACC = 1, R_RESTART = 0 };
-enum Bug { B_NONE, B_PUBLISH_EARLY, B_RESUME_SKIP, B_NO_RELEASE, B_NO_GATE, B_DOUBLE_SERVE };
+enum Bug { B_NONE, B_PUBLISH_EARLY, B_RESUME_SKIP, B_NO_RELEASE, B_NO_GATE, B_DOUBLE_SERVE,
+           B_DUE_BOTH };
 
 struct Config {
   bool retreat = false;
@@ -372,18 +382,51 @@ Bug parse_bug(const std::string& s) {
   if (s == "no-release") return B_NO_RELEASE;
   if (s == "no-gate") return B_NO_GATE;
   if (s == "double-serve") return B_DOUBLE_SERVE;
+  if (s == "due-both") return B_DUE_BOTH;
   return B_NONE;
+}
+
+// The setter block's waves over 10,000 poll sites, random clocks and schedules.
+int setter_arm(unsigned seed, int waves, Bug bug) {
+  std::mt19937 rng(seed);
+  int due[2] = {1, 1};
+  std::vector<proto::SetterLook<HostPlat>> look((size_t)waves,
+                                                proto::SetterLook<HostPlat>{due, 0});
+  std::vector<int> order((size_t)waves);
+  for (int w = 0; w < waves; ++w) order[(size_t)w] = w;
+  long split = 0, left = 0;
+  for (int site = 0; site < 10000; ++site) {
+    std::shuffle(order.begin(), order.end(), rng);
+    int agreed = -1;
+    for (int w : order) {  // one wave from this site's barrier to the next
+      auto& l = look[(size_t)w];
+      const bool d = l.at_site(w == 0, [&] { return rng() % 3 == 0; });
+      if (d && w == 0) {  // out of the loop, with no barrier: an event is raised
+        const bool again = rng() % 2 == 0;
+        l.next(again);
+        if (bug == B_DUE_BOTH) due[0] = due[1] = again;
+      }
+      if (agreed >= 0 && (int)d != agreed) ++split;
+      agreed = (int)d;
+      left += w == 0 && d;
+    }
+  }
+  printf("%s: setter waves %d left %ld split %ld\n", split ? "FAIL" : "PASS", waves, left, split);
+  return split ? 1 : 0;
 }
 
 }  // namespace
 
 int main(int argc, char** argv) {
   Config c;
+  bool setter = false;
+  int waves = 4;
   std::string bug = "none";
   for (int i = 1; i + 1 < argc; i += 2) {
     const std::string k = argv[i];
     const char* v = argv[i + 1];
-    if (k == "--arm") c.retreat = std::string(v) == "retreat";
+    if (k == "--arm") c.retreat = std::string(v) == "retreat", setter = std::string(v) == "setter";
+    else if (k == "--waves") waves = atoi(v);
     else if (k == "--blocks") c.blocks = atoi(v);
     else if (k == "--tiles-m") c.tilesM = atoi(v);
     else if (k == "--tiles-n") c.tilesN = atoi(v);
@@ -411,6 +454,7 @@ int main(int argc, char** argv) {
     }
   }
   c.bug = parse_bug(bug);
+  if (setter && waves > 0) return setter_arm(c.seed, waves, c.bug);
   if (c.blocks < 1 || c.stages < 2 || c.events < 0 || c.pollEvery < 1 || c.domains < 1 ||
       c.domains > APK_RETREAT_DOMAINS || c.urgentTiles < 1 || c.tilesM < 1 || c.tilesN < 1 ||
       c.passes < 1 || (c.cap != 0 && c.cap < 2) || c.rqWaitTicks < 0 || c.urgentNs < 0 ||

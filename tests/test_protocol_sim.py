@@ -214,3 +214,18 @@ def test_queue_hands_out_every_task_once(batch, statics, blocks, tiles_m, tiles_
                       "--batch", batch, "--statics", statics, job=False)
     assert rc == 0 and line.startswith("PASS"), line
     assert f["dup"] == 0 and f["miss"] == 0, line
+
+
+@pytest.mark.parametrize("waves", [1, 4, 8])
+def test_setter_waves_agree(waves):
+    """Every wave of the setter block decides alike at every poll site, in
+    whatever order the waves run between two barriers."""
+    rc, line, f = run("--arm", "setter", "--waves", waves, "--seed", 3, job=False)
+    assert rc == 0 and f["split"] == 0 and f["left"] > 100, line
+
+
+def test_setter_write_to_the_word_being_read_is_caught():
+    """Thread 0 writing, with no barrier, the word that other waves may still
+    be reading at the same site splits the block."""
+    rc, line, f = run("--arm", "setter", "--seed", 3, "--bug", "due-both", job=False)
+    assert rc == 1 and f["split"] > 0, line
