@@ -5,7 +5,9 @@
 // The fp32 matrix instructions give 157 TFLOP/s, the bf16 ones sixteen times
 // that. Each operand is therefore split into three bf16 parts, x = hi + mid +
 // lo, every part the round-to-nearest bf16 of what the former leave: 24
-// significand bits in all, so x is represented exactly. A product is the sum
+// significand bits in all, so x is represented exactly down to bf16's last bit
+// (2^-133; the conversions and v_mfma_f32_32x32x16_bf16 keep denormals, in
+// operands, products and sums). A product is the sum
 // of the six part products down to 2^-16 of hi.hi (the three left out are
 // below 2^-24 of it), accumulated in fp32 by v_mfma_f32_32x32x16_bf16, which
 // rounds once per 8 products where the fp32 instructions round at every one.
@@ -14,8 +16,8 @@
 // What the parts cannot carry is computed with exact fp32 products instead
 // (suspect, compute_exact): tiles with an infinite or NaN accumulator (an
 // operand or a sum that is infinite, NaN, or above bf16's largest value) and
-// tiles with an operand below 2^-100 other than zero (its lowest part could
-// be rounded).
+// tiles with an operand that has bits below 2^-133 (below 2^-110, that is),
+// which its parts lose.
 //
 // Block: 256 threads = 4 wave64s in a 2x2 arrangement; each wave owns a
 // 64x64 sub-tile held as 2x2 32x32 accumulators (64 VGPRs per lane).
@@ -60,7 +62,6 @@ namespace apk {
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 struct EngMfma128 {
   static constexpr int TM = 128, TN = 128, KS = 32, NS = 3, GROUP = 1, THREADS = 256;
@@ -85,7 +86,7 @@ struct EngMfma128 {
 
   struct Acc {
     f32x16 c[2][2];
-    u16x2 tiny;  // smallest operands seen (tiny_watch)
+    unsigned rest;  // what the last parts were rounded from, all or'ed (split_part)
   };
 
   static __device__ __forceinline__ int aswz(int r) { return (r ^ ((r >> 3) & 1)) & 7; }
@@ -113,7 +114,7 @@ struct EngMfma128 {
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) a.c[i][j][r] = 0.0f;
-    a.tiny = u16x2{0xffff, 0xffff};
+    a.rest = 0;
   }
 
   // Direct-to-LDS loads of one k-stage. A load i (< 4) fills the 1 KiB
@@ -180,8 +181,8 @@ struct EngMfma128 {
   // block (the quad 2g+h of the lane's row), four B dwords per 32-column
   // block (compute_exact). The wave's blocks are numbered so that block 0 of A is another
   // one for its neighbour in the column, and block 0 of B for its neighbour
-  // in the row (arow, bcol): each wave watches its blocks 0 for small
-  // operands (tiny_watch), and together the four watch every operand once.
+  // in the row (arow, bcol): each wave splits its blocks 0, and together the
+  // four split every operand once.
   struct Frag {
     f32x4 a4[2];
     float bv[2][4];
@@ -267,8 +268,9 @@ struct EngMfma128 {
       rest = Rest{rest.x0 - low(mid), rest.x1 - high(mid)};
       o[1][p & 3] = mid;
     } else {
+      // bf16 is the upper half of fp32: lo is exact where the lower is zero.
       o[2][p & 3] = pack(rest.x0, rest.x1);
-      tiny_watch(o[0][p & 3], acc);
+      acc.rest |= __float_as_uint(rest.x0) | __float_as_uint(rest.x1);
     }
   }
   // This lane's 16 bytes of plane 0 of block `blk` (0-3 A's rows, 4-7 B's
@@ -294,13 +296,6 @@ struct EngMfma128 {
   static __device__ __forceinline__ float low(unsigned u) { return __uint_as_float(u << 16); }
   static __device__ __forceinline__ float high(unsigned u) {
     return __uint_as_float(u & 0xffff0000u);
-  }
-  // Keeps the smallest non-zero magnitude seen, as twice the bf16 bits less
-  // one (the sign falls out, and zero wraps to the largest value).
-  static __device__ __forceinline__ void tiny_watch(unsigned hi, Acc& acc) {
-    unsigned t;  // both halves: 2 x - 1
-    asm("v_pk_mad_u16 %0, %1, 2, -1 op_sel_hi:[1,0,1]" : "=v"(t) : "v"(hi));
-    acc.tiny = __builtin_elementwise_min(acc.tiny, __builtin_bit_cast(u16x2, t));
   }
   // MFMA m (< 24) of a k-step. Blocks in the order (own, own), (own, other),
   // (other, own), (other, other), each with its six products in ascending
@@ -398,10 +393,9 @@ struct EngMfma128 {
 
   // Whether the tile must be computed again with exact products (this lane):
   // a non-finite accumulator -- an operand or a sum was infinite, NaN or
-  // beyond bf16's largest value --, or an operand whose lowest bits bf16 may
-  // not hold (below 2^-100; lo's last bit of anything larger is a normal
-  // number).
-  static constexpr unsigned short TINY = 2 * ((127 - 100) << 7) - 1;
+  // beyond bf16's largest value --, or an operand that is more than its
+  // parts.
+  static __device__ __forceinline__ bool lossy(const Acc& a) { return (a.rest & 0xffffu) != 0; }
   static __device__ __forceinline__ bool suspect(const Acc& a) {
     float z[2] = {0.0f, 0.0f};
 #pragma unroll
@@ -410,7 +404,7 @@ struct EngMfma128 {
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) z[j] = fmaf(a.c[i][j][r], 0.0f, z[j]);
-    return !(z[0] + z[1] == 0.0f) || a.tiny[0] < TINY || a.tiny[1] < TINY;
+    return !(z[0] + z[1] == 0.0f) || lossy(a);
   }
   // One k-stage with the exact fp32 products of v_mfma_f32_32x32x2_f32 (the
   // path of tiles with suspect() operands).
@@ -440,14 +434,14 @@ struct EngMfma128 {
     r = arow(rb) + 8 * (q >> 2) + 4 * (l >> 5) + (q & 3);
     c = bcol(cb) + (l & 31);
   }
-  // A checkpoint carries `tiny` as a NaN in the lane's first accumulator: the
+  // A checkpoint carries lossy() as a NaN in the lane's first accumulator: the
   // resumed tile then ends suspect, as this one would have.
   static __device__ __forceinline__ float get(const Acc& a, int e) {
-    if (e == 0 && (a.tiny[0] < TINY || a.tiny[1] < TINY)) return __builtin_nanf("");
+    if (e == 0 && lossy(a)) return __builtin_nanf("");
     return a.c[e >> 5][(e >> 4) & 1][e & 15];
   }
   static __device__ __forceinline__ void set(Acc& a, int e, float v) {
-    if (e == 0) a.tiny = u16x2{0xffff, 0xffff};
+    if (e == 0) a.rest = 0;
     a.c[e >> 5][(e >> 4) & 1][e & 15] = v;
   }
 

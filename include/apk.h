@@ -35,7 +35,7 @@ enum {
  *             three bf16 parts and multiplied by v_mfma_f32_32x32x16_bf16 with
  *             fp32 accumulation (error against 64 bits below the fp32 chain's);
  *             tiles with operands or sums that bf16's range cannot carry
- *             (infinite, NaN, above 3.39e38, below 2^-100) are computed with
+ *             (infinite, NaN, above 3.39e38, bits below 2^-133) are computed with
  *             v_mfma_f32_32x32x2_f32 products.
  *  BF16X256 : 256x256 tile of a bf16 GEMM with fp32 accumulation on
  *             v_mfma_f32_32x32x16_bf16, 512 threads (two waves per SIMD),

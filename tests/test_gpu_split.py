@@ -1,6 +1,6 @@
 """The fp32 MFMA tile's split products (three bf16 parts per operand) on the
 GPU: no less exact than the fp32 chain over the range of K, and operands that
-the parts cannot carry (infinite, NaN, above bf16's range, below 2^-100)
+the parts cannot carry (infinite, NaN, above bf16's range, bits below 2^-133)
 computed with exact products, also through checkpoint and resume.
 
 Bound for finite results: each C element sums K products in fp32, at most K
@@ -112,3 +112,57 @@ def test_split_special_operands_through_yields(torch_gpu, apk, kind, resume):
     if kind == "tiny_one":
         ref = j.A.astype(np.float64) @ j.B.astype(np.float64)
         assert (np.abs(off["C"] - ref) <= _bound(j.A[:, :8], j.B[:8])).all()
+
+
+# An operand alone in its row (column): all that its outputs hold. 2^-134 and
+# below round to a bf16 zero; from 2^-110 on the three parts hold every bit.
+@pytest.mark.parametrize("exp", [-149, -141, -135, -134, -133, -127, -112, -109, -90])
+@pytest.mark.parametrize("side", ["A", "B"])
+def test_split_small_operand_alone(torch_gpu, apk, side, exp):
+    say(f"mfma128 small operand 2^{exp} alone in {side}")
+    A, B = oracle.fill_uniform_pm1(7, 256, 256, 96)
+    x = np.float32(-1.2345678 * 2.0 ** exp)
+    if side == "A":
+        A[200] = 0
+        A[200, 70] = x
+        B *= np.float32(2.0 ** 100)
+    else:
+        B[:, 33] = 0
+        B[5, 33] = x
+        A *= np.float32(2.0 ** 100)
+    C, _, _ = run_persistent(torch_gpu, apk, apk.ENGINE_MFMA128, A, B, 96, blocks=3,
+                             with_log=False)
+    ref = A.astype(np.float64) @ B.astype(np.float64)
+    alone = ref[200] if side == "A" else ref[:, 33]
+    assert (np.abs(alone) > 0).all()  # a lost operand leaves zeros, far outside the bound
+    assert (np.abs(C - ref) <= _bound(A, B)).all()
+
+
+# Ordinary operands whose products and sums (or only the parts' products) are
+# denormal, and operands over a wide range of exponents.
+@pytest.mark.parametrize("ea,eb", [(-62, -62), (-70, -70), (-72, -73), (-100, -20)])
+def test_split_denormal_sums(torch_gpu, apk, ea, eb):
+    say(f"mfma128 operands of 2^{ea} and 2^{eb}")
+    A, B = oracle.fill_uniform_pm1(9, 256, 256, 96)
+    A *= np.float32(2.0 ** ea)
+    B *= np.float32(2.0 ** eb)
+    C, _, _ = run_persistent(torch_gpu, apk, apk.ENGINE_MFMA128, A, B, 96, blocks=3,
+                             with_log=False)
+    ref = A.astype(np.float64) @ B.astype(np.float64)
+    assert (np.abs(C - ref) <= _bound(A, B)).all()
+
+
+@pytest.mark.parametrize("K", [64, 992])
+def test_split_wide_exponents(torch_gpu, apk, K):
+    say(f"mfma128 wide exponents K={K}")
+    rng = np.random.default_rng(3)
+    A, B = oracle.fill_uniform_pm1(11, 256, 256, K)
+    A *= np.exp2(rng.integers(-30, 30, A.shape)).astype(np.float32)
+    B *= np.exp2(rng.integers(-30, 30, B.shape)).astype(np.float32)
+    C, _, _ = run_persistent(torch_gpu, apk, apk.ENGINE_MFMA128, A, B, K, blocks=3,
+                             with_log=False)
+    ref = oracle.gemm_f64(A, B, threads=8)
+    err, err_chain = oracle.rel_frobenius(C, ref), oracle.rel_frobenius(
+        oracle.gemm_f32_chain(A, B), ref)
+    say(f"  rel-Frobenius {err:.2e}, fp32 chain {err_chain:.2e}")
+    assert (np.abs(C - ref) <= _bound(A, B)).all()
