@@ -405,7 +405,7 @@ struct EngBf16T {
     return true;
   }
   // The last pair's deferred MFMAs, before the accumulators are read.
-  static __device__ __forceinline__ void finish_tail(const char*, Acc& acc, const Tail& tail) {
+  static __device__ __forceinline__ void finish_tail(Acc& acc, const Tail& tail) {
 #pragma unroll
     for (int m = 0; m < NT_MF; ++m) {
       const int rb = m / CB, cb = m % CB;

@@ -14,10 +14,16 @@
 // Error against 64 bits, uniform [-1, 1) operands, K = 256 / 992 / 4096:
 // 2.3e-7 / 4.8e-7 / 1.0e-6 (fp32 chain 2.9e-7 / 5.6e-7 / 1.1e-6).
 // What the parts cannot carry is computed with exact fp32 products instead
-// (suspect, compute_exact): tiles with an infinite or NaN accumulator (an
-// operand or a sum that is infinite, NaN, or above bf16's largest value) and
-// tiles with an operand that has bits below 2^-133 (below 2^-110, that is),
-// which its parts lose.
+// (compute_exact, at the fp32 matrix rate and with the same poll sites):
+//  - from the first k-stage on that holds an operand with bits below 2^-133
+//    (below 2^-110, that is), which its parts lose, to the end of the tile;
+//  - a tile that ends with an infinite or NaN accumulator (an operand or a sum
+//    that is infinite, NaN, or above bf16's largest value), from k = 0.
+// Both are decided by the tile's operands alone, so a tile's result does not
+// depend on where it was checkpointed. 4096^3, with fp32 products throughout
+// 975 us: ordinary operands 790, softmax weights (two fifths of them below
+// 2^-110) 1037, all 1e-35 1020, one small operand per panel in the middle of K
+// 880; an infinity at k = 0 1060-1100, a NaN at the end of K 1740 (both passes).
 //
 // Block: 256 threads = 4 wave64s in a 2x2 arrangement; each wave owns a
 // 64x64 sub-tile held as 2x2 32x32 accumulators (64 VGPRs per lane).
@@ -86,7 +92,6 @@ struct EngMfma128 {
 
   struct Acc {
     f32x16 c[2][2];
-    unsigned rest;  // what the last parts were rounded from, all or'ed (split_part)
   };
 
   static __device__ __forceinline__ int aswz(int r) { return (r ^ ((r >> 3) & 1)) & 7; }
@@ -114,7 +119,6 @@ struct EngMfma128 {
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) a.c[i][j][r] = 0.0f;
-    a.rest = 0;
   }
 
   // Direct-to-LDS loads of one k-stage. A load i (< 4) fills the 1 KiB
@@ -148,15 +152,6 @@ struct EngMfma128 {
   struct Dst {
     uint32_t lds, ka, kb;
   };
-  // Materialises a stage's load descriptors in scalar registers at this
-  // point of the program (nothing moves their computation later). They are
-  // uniform by construction; readfirstlane only tells the compiler so.
-  static __device__ __forceinline__ void pin(Dst& d) {
-    d.lds = __builtin_amdgcn_readfirstlane(d.lds);
-    d.ka = __builtin_amdgcn_readfirstlane(d.ka);
-    d.kb = __builtin_amdgcn_readfirstlane(d.kb);
-    asm volatile("" : "+s"(d.lds), "+s"(d.ka), "+s"(d.kb));
-  }
   // A stage past the tile's end (t >= S) fetches stage S-1 again: nothing
   // reads that slot before it is refilled.
   static __device__ __forceinline__ Dst stage_dst(uint32_t wave_lds, const Ctx& c, int slot,
@@ -253,8 +248,9 @@ struct EngMfma128 {
   struct Rest {
     float x0, x1;
   };
+  // `seen` collects what the lowest parts were rounded from (lossy).
   static __device__ __forceinline__ void split_part(const Raw& r, int part, Own& d, Rest& rest,
-                                                    Acc& acc) {
+                                                    unsigned& seen) {
     const int p = part / 3, e = 2 * (p & 3);  // elements e, e + 1
     u32x4* o = p < 4 ? d.a : d.b;
     if (part % 3 == 0) {
@@ -268,9 +264,8 @@ struct EngMfma128 {
       rest = Rest{rest.x0 - low(mid), rest.x1 - high(mid)};
       o[1][p & 3] = mid;
     } else {
-      // bf16 is the upper half of fp32: lo is exact where the lower is zero.
       o[2][p & 3] = pack(rest.x0, rest.x1);
-      acc.rest |= __float_as_uint(rest.x0) | __float_as_uint(rest.x1);
+      seen |= __float_as_uint(rest.x0) | __float_as_uint(rest.x1);
     }
   }
   // This lane's 16 bytes of plane 0 of block `blk` (0-3 A's rows, 4-7 B's
@@ -323,27 +318,77 @@ struct EngMfma128 {
     Own own;
     Raw raw;
   };
-  // The MFMAs of the step whose own blocks are `cur` (the others' in planes
-  // `buf`); under them `raw` is split into `next` and planes buf ^ 1 (SPLIT),
-  // and `mid(i)`, i = lo..lo+3, issues loads (four of them).
-  template <bool SPLIT, class Read, class Mid>
-  static __device__ __forceinline__ void phase(char* ring, int buf, const Own& cur,
-                                               const Raw& raw, Own& next, Acc& acc, Read&& read,
-                                               int lo, Mid&& mid) {
-    Own other;
-    Rest rest;
-    take(plane(ring, buf, bblock(1)), other.b);
-    take(plane(ring, buf, ablock(1)), other.a);
+  // How a tile is computed: with parts; from some stage on with exact
+  // products; with exact products throughout. And what the stage whose MFMAs
+  // are next turned out to be: LOSSY, it holds an operand that is more than
+  // its parts; BROKEN, an accumulator is infinite or NaN already.
+  enum { SPLIT = 0, EXACT_REST = 1, EXACT = 2 };
+  enum { FINE = 0, LOSSY = 1, BROKEN = 2 };
+
+  // Whether this lane's operands of a stage are more than their parts. Its
+  // first k-step has been split: bf16 is the upper half of fp32, so lo is
+  // exact where the lower half of what it was rounded from (`seen`) is zero.
+  // The second has only been read (its MFMAs, like the first's, come after
+  // the next barrier, and the stage's slot is refilled after that): `least`
+  // is the smallest of 2 |x| - 1 as an integer, where a zero wraps to the
+  // largest, and 2^-110 the smallest normal value without bits below 2^-133.
+  static constexpr unsigned LEAST = 2u * ((127 - 110) << 23) - 1;
+  static __device__ __forceinline__ bool lossy(unsigned seen, unsigned least) {
+    return (seen & 0xffffu) != 0 || least < LEAST;
+  }
+  static __device__ __forceinline__ void watch(const Raw& r, int p, unsigned& least) {
+    const int e = 2 * (p & 3);
+    const unsigned x0 = __float_as_uint(p < 4 ? r.a[e >> 2][e & 3] : r.b[e]);
+    const unsigned x1 = __float_as_uint(p < 4 ? r.a[e >> 2][(e & 3) + 1] : r.b[e + 1]);
+    const unsigned t0 = 2 * x0 - 1, t1 = 2 * x1 - 1;
+    const unsigned t = t0 < t1 ? t0 : t1;
+    least = t < least ? t : least;
+  }
+  // A lane of the block marks stage s: verdict[s & 1] (LDS, both words zero
+  // when the tile starts) is read after the next barrier. Two words: a wave
+  // ahead of the others marks stage s + 1 while they still read s's.
+  // Every 16 stages it also looks for a sum that is no longer finite, so that
+  // a tile of infinite or NaN operands does not run to its end first: one
+  // register per column block and every one of column block 0 meet any row
+  // or column of them.
+  static __device__ __forceinline__ void mark(int* verdict, int s, unsigned seen, unsigned least,
+                                              const Acc& acc) {
+    if (lossy(seen, least)) verdict[s & 1] = LOSSY;
+    if ((s & 15) == 15) {
+      float z = acc.c[0][1][0] * 0.0f;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) z = fmaf(acc.c[i][0][r], 0.0f, z);
+      if (!(z == 0.0f)) verdict[s & 1] = BROKEN;
+    }
+  }
+  // Stage s's verdict, after the barrier that follows its call (uniform).
+  static __device__ __forceinline__ int verdict_of(const int* verdict, int s) {
+    return uniform(verdict[s & 1]);
+  }
+
+  static __device__ __forceinline__ void take_other(const char* ring, int buf, Own& other) {
+    take(plane(const_cast<char*>(ring), buf, bblock(1)), other.b);
+    take(plane(const_cast<char*>(ring), buf, ablock(1)), other.a);
     __builtin_amdgcn_sched_barrier(0);
+  }
+  // The MFMAs of the step whose blocks are `cur` and `other`; under MFMA m part
+  // m of `raw` is split into `next` and planes `buf` (SPLIT_NEXT), `at(m)`
+  // runs, and `mid(i)`, i = lo..lo+3, issues loads (four of them).
+  template <bool SPLIT_NEXT, class At, class Mid>
+  static __device__ __forceinline__ void phase(char* ring, int buf, const Own& cur,
+                                               const Own& other, const Raw& raw, Own& next,
+                                               unsigned& seen, Acc& acc, At&& at, int lo,
+                                               Mid&& mid) {
+    Rest rest;
 #pragma unroll
     for (int m = 0; m < MF; ++m) {
       mma(cur, other, m, acc);
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (SPLIT) split_put(ring, buf ^ 1, raw, m, next, rest, acc);
-      if (m == 6) {
-        read();
-        __builtin_amdgcn_sched_barrier(0);
-      }
+      if constexpr (SPLIT_NEXT) split_put(ring, buf, raw, m, next, rest, seen);
+      at(m);
+      __builtin_amdgcn_sched_barrier(0);
       if (m % 5 == 4 && m / 5 < LOADS / 2) {
         mid(lo + m / 5);
         __builtin_amdgcn_sched_barrier(0);
@@ -352,51 +397,80 @@ struct EngMfma128 {
   }
   // Part `part`; a block goes to the planes once its last part is done.
   static __device__ __forceinline__ void split_put(char* ring, int buf, const Raw& raw, int part,
-                                                   Own& d, Rest& rest, Acc& acc) {
-    split_part(raw, part, d, rest, acc);
+                                                   Own& d, Rest& rest, unsigned& seen) {
+    split_part(raw, part, d, rest, seen);
     if (part == 11) put(plane(ring, buf, ablock(0)), d.a);
     if (part == 23) put(plane(ring, buf, bblock(0)), d.b);
     __builtin_amdgcn_sched_barrier(0);
   }
-  // Stage `slot` of the ring enters the pipeline; the two steps before it
-  // leave it (hasTail = false: there are none). `mid(i)`, i = 0..LOADS-1,
-  // issues the loads of a later stage, spread over the MFMAs.
+  // Stage s in ring slot `slot` enters the empty pipeline. `mid(i)`, i =
+  // 0..LOADS-1, issues the loads of a later stage.
   template <class Mid>
-  static __device__ __forceinline__ void stage(char* ring, int slot, Acc& acc, Tail& t,
-                                               bool hasTail, Mid&& mid) {
+  static __device__ __forceinline__ void enter(char* ring, int slot, int s, const Acc& acc,
+                                               Tail& t, int* verdict, Mid&& mid) {
+    const char* abase = ring + slot * STAGE;
+    Raw raw;
+    Rest rest;
+    unsigned seen = 0, least = ~0u;
+    load_raw(abase, 0, raw);
+    load_raw(abase, 1, t.raw);
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) mid(i);
+#pragma unroll
+    for (int p = 0; p < MF; ++p) split_put(ring, 0, raw, p, t.own, rest, seen);
+#pragma unroll
+    for (int p = 0; p < 8; ++p) watch(t.raw, p, least);
+    mark(verdict, s, seen, least, acc);
+  }
+  // Stage s in ring slot `slot` enters the pipeline and the two steps of stage
+  // s - 1 leave it; `mid`'s loads are spread over their MFMAs. If stage s - 1
+  // is not FINE, its verdict is returned (uniform), with nothing done. The
+  // verdict is read ahead of the planes, whose reads cover most of its way:
+  // looking for lossy stages costs 4096^3 0.7%, a 256^3 urgent job 14.0 ->
+  // 14.4 us.
+  template <class Mid>
+  static __device__ __forceinline__ int stage(char* ring, int slot, int s, Acc& acc, Tail& t,
+                                              int* verdict, Mid&& mid) {
     static_assert(STEPS == 2 && LOADS == 8, "two phases per stage, four loads each");
     const char* abase = ring + slot * STAGE;
     Raw raw;
-    if (hasTail) {
-      Own odd;
-      phase<true>(ring, 0, t.own, t.raw, odd, acc, [&] { load_raw(abase, 0, raw); }, 0, mid);
-      lds_sync();
-      phase<true>(ring, 1, odd, raw, t.own, acc, [&] { load_raw(abase, 1, t.raw); }, 4, mid);
-    } else {
-      Rest rest;
-      load_raw(abase, 0, raw);
-      load_raw(abase, 1, t.raw);
-#pragma unroll
-      for (int i = 0; i < LOADS; ++i) mid(i);
-#pragma unroll
-      for (int p = 0; p < MF; ++p) split_put(ring, 0, raw, p, t.own, rest, acc);
-    }
-  }
-  // The two steps left over, before the accumulators are read.
-  static __device__ __forceinline__ void finish_tail(char* ring, Acc& acc, const Tail& t) {
-    Own odd;
-    lds_sync();  // every wave's planes
-    phase<true>(ring, 0, t.own, t.raw, odd, acc, [] {}, 0, [](int) {});
+    unsigned seen = 0, unused = 0, least = ~0u;
+    const int v = verdict[(s - 1) & 1];
+    __builtin_amdgcn_sched_barrier(0);
+    Own odd, other;
+    take_other(ring, 0, other);
+    if (const int u = uniform(v)) return u;
+    phase<true>(ring, 1, t.own, other, t.raw, odd, unused, acc,
+                   [&](int m) { if (m == 6) load_raw(abase, 0, raw); }, 0, mid);
     lds_sync();
-    phase<false>(ring, 1, odd, t.raw, odd, acc, [] {}, 0, [](int) {});
+    take_other(ring, 1, other);
+    phase<true>(ring, 0, odd, other, raw, t.own, seen, acc,
+                   [&](int m) {
+                     if (m == 6) load_raw(abase, 1, t.raw);
+                     if (m >= 9 && m % 2) watch(t.raw, (m - 9) / 2, least);
+                   },
+                   4, mid);
+    mark(verdict, s, seen, least, acc);
+    return FINE;
+  }
+  // The two steps left over of stage s, before the accumulators are read;
+  // with nothing done but a barrier if the stage is not FINE.
+  static __device__ __forceinline__ int finish_tail(char* ring, int s, Acc& acc, const Tail& t,
+                                                    const int* verdict) {
+    Own odd, other;
+    unsigned unused = 0;
+    lds_sync();  // every wave's planes and verdict
+    if (const int u = verdict_of(verdict, s)) return u;
+    take_other(ring, 0, other);
+    phase<true>(ring, 1, t.own, other, t.raw, odd, unused, acc, [](int) {}, 0, [](int) {});
+    lds_sync();
+    take_other(ring, 1, other);
+    phase<false>(ring, 0, odd, other, t.raw, odd, unused, acc, [](int) {}, 0, [](int) {});
+    return FINE;
   }
 
-  // Whether the tile must be computed again with exact products (this lane):
-  // a non-finite accumulator -- an operand or a sum was infinite, NaN or
-  // beyond bf16's largest value --, or an operand that is more than its
-  // parts.
-  static __device__ __forceinline__ bool lossy(const Acc& a) { return (a.rest & 0xffffu) != 0; }
-  static __device__ __forceinline__ bool suspect(const Acc& a) {
+  // Whether an accumulator of this lane is infinite or NaN.
+  static __device__ __forceinline__ bool broken(const Acc& a) {
     float z[2] = {0.0f, 0.0f};
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -404,11 +478,14 @@ struct EngMfma128 {
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) z[j] = fmaf(a.c[i][j][r], 0.0f, z[j]);
-    return !(z[0] + z[1] == 0.0f) || lossy(a);
+    return !(z[0] + z[1] == 0.0f);
   }
-  // One k-stage with the exact fp32 products of v_mfma_f32_32x32x2_f32 (the
-  // path of tiles with suspect() operands).
-  static __device__ __forceinline__ void compute_exact(const char* ring, int slot, Acc& acc) {
+  // One k-stage with the exact fp32 products of v_mfma_f32_32x32x2_f32. The
+  // operands of group g+1 are read from LDS while group g's MFMAs run;
+  // `mid(i)`, i < LOADS, issues a later stage's loads under the first ones.
+  template <class Mid>
+  static __device__ __forceinline__ void compute_exact(const char* ring, int slot, Acc& acc,
+                                                       Mid&& mid) {
     const char* abase = ring + slot * STAGE;
     constexpr int GG = KS / 8;
     Frag f[2];
@@ -423,6 +500,11 @@ struct EngMfma128 {
         const int s = m >> 2, rb = (m >> 1) & 1, cb = m & 1;
         acc.c[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(c.a4[rb][s], c.bv[cb][s],
                                                              acc.c[rb][cb], 0, 0, 0);
+        if ((m & 1) && g * 8 + (m >> 1) < LOADS) {
+          __builtin_amdgcn_sched_barrier(0);
+          mid(g * 8 + (m >> 1));
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
     }
   }
@@ -434,14 +516,10 @@ struct EngMfma128 {
     r = arow(rb) + 8 * (q >> 2) + 4 * (l >> 5) + (q & 3);
     c = bcol(cb) + (l & 31);
   }
-  // A checkpoint carries lossy() as a NaN in the lane's first accumulator: the
-  // resumed tile then ends suspect, as this one would have.
   static __device__ __forceinline__ float get(const Acc& a, int e) {
-    if (e == 0 && lossy(a)) return __builtin_nanf("");
     return a.c[e >> 5][(e >> 4) & 1][e & 15];
   }
   static __device__ __forceinline__ void set(Acc& a, int e, float v) {
-    if (e == 0) a.rest = 0;
     a.c[e >> 5][(e >> 4) & 1][e & 15] = v;
   }
 

@@ -26,7 +26,7 @@ __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu
   __shared__ __attribute__((aligned(16))) char ring[E::LDS_BYTES];
   __shared__ unsigned s_task;
   __shared__ proto::QueueCursor s_cur;  // thread 0's place in the queue
-  __shared__ int s_suspect;
+  __shared__ int s_verdict[VERDICT_WORDS];
 
   const int tilesN = N / E::TN;
   const unsigned numTasks = (unsigned)((M / E::TM) * tilesN);
@@ -38,7 +38,7 @@ __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu
   const typename E::Ctx ctx = E::make_ctx(A, B, M, N, K);
   const uint32_t wl = wave_lds(ring);
   if (threadIdx.x == 0) {
-    s_suspect = 0;
+    s_verdict[2] = 0;
     s_cur = proto::QueueCursor{0, 0, 0, 0, 0};
     tq.start(s_cur, blockIdx.x);
   }
@@ -64,7 +64,7 @@ __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu
     // one uniform compare per stage instead of a modulo under a per-thread
     // branch at the top of every stage.
     int nextRec = rec ? 0 : INT_MAX;
-    run_stages<E>(ring, wl, ctx, acc, row0, col0, K / E::KS, &s_suspect, [&](int s) {
+    run_stages<E>(ring, wl, ctx, acc, row0, col0, K / E::KS, s_verdict, [&](int s) {
       if (s != nextRec) return;
       nextRec += spc;
       if (threadIdx.x == 0) {
@@ -108,15 +108,15 @@ __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu
                    unsigned long long* end_gt) {
   if (start_gt && blockIdx.x == 0 && threadIdx.x == 0) *start_gt = (long long)wall_ticks();
   __shared__ __attribute__((aligned(16))) char ring[E::LDS_BYTES];
-  __shared__ int s_suspect;
-  if (threadIdx.x == 0) s_suspect = 0;  // first read after a stage's barrier
+  __shared__ int s_verdict[VERDICT_WORDS];
+  if (threadIdx.x == 0) s_verdict[2] = 0;  // first read after a stage's barrier
   const int tilesN = N / E::TN;
   const int row0 = (int)(blockIdx.x / (unsigned)tilesN) * E::TM;
   const int col0 = (int)(blockIdx.x % (unsigned)tilesN) * E::TN;
   const typename E::Ctx ctx = E::make_ctx(A, B, M, N, K);
   typename E::Acc acc;
   E::zero(acc);
-  run_stages<E>(ring, wave_lds(ring), ctx, acc, row0, col0, K / E::KS, &s_suspect, [](int) {});
+  run_stages<E>(ring, wave_lds(ring), ctx, acc, row0, col0, K / E::KS, s_verdict, [](int) {});
   store_tile<E>(acc, ring, C, N, row0, col0, false);
   if (end_gt) {
     wait_vmcnt<0>();  // this thread's C stores have completed

@@ -61,7 +61,7 @@ k_persistent_yield(const apk_yield_params) {
   __shared__ long long s_serve_t1;   // start of the current service's urgent work
   __shared__ int s_fsync;            // synchronous flag read (syncPoll)
   __shared__ proto::QueueCursor s_cur;  // thread 0's place in the work queue
-  __shared__ int s_suspect;          // a lane ended its tile suspect (note_suspect)
+  __shared__ int s_verdict[VERDICT_WORDS];  // split operands (pipeline.hpp)
 
   const int tid = threadIdx.x, bid = blockIdx.x;
   // Values the stage loop does not need are recomputed from the parameters
@@ -137,7 +137,7 @@ k_persistent_yield(const apk_yield_params) {
   if (tid < 2) s_due[tid] = 1;  // the first site sets the time base
   if (tid == 0) {
     s_cur = proto::QueueCursor{0, 0, 0, 0, 0};
-    s_suspect = 0;
+    s_verdict[2] = 0;
   }
   if (P().run_gt && bid == 0 && tid == 0) P().run_gt[0] = wall_ticks();
   __syncthreads();
@@ -214,12 +214,15 @@ k_persistent_yield(const apk_yield_params) {
   // checkpoint. Urgent tiles go through the same loop, so the kernel holds
   // one software pipeline and one epilogue, not two of each.
   enum { FRESH = 0, ACC = 1, FULL = 2, AS_IS = 3 };
+  // A resume entry's stage word: the stage, and above it the tile's mode.
+  constexpr int RQ_MODE_SHIFT = 28, RQ_STAGE = (1 << RQ_MODE_SHIFT) - 1;
   int serving = -1;        // event this block serves, or -1
   int uidx = 0;            // while serving: the urgent tile of the next job
   unsigned savedTask = 0;  // while serving: the interrupted background task,
   int savedStage = 0;      // its stage and how it re-enters
   int savedSite = 0;       // the site it left
   int savedKind = FRESH;
+  int savedMode = 0;       // and how it is computed (E::SPLIT, ...)
 
   for (;;) {
     // host stop sentinel: no task is taken any more (one taken with an
@@ -248,6 +251,7 @@ k_persistent_yield(const apk_yield_params) {
     int srcKind = FRESH, s = 0, siteDone = -1;
     const float* src = nullptr;
     bool urgent = false;
+    int mode = 0;     // uniform; split operands: E::SPLIT, E::EXACT_REST, E::EXACT
     int rqHeld = -1;  // resume ticket whose checkpoint this job reads back
     bool startSite = false;  // uniform: a task-start sample was taken for this job
     int fStart = 0;          // uniform: its value
@@ -269,6 +273,7 @@ k_persistent_yield(const apk_yield_params) {
         if (savedKind != FRESH) {
           s = savedStage;
           siteDone = savedSite;
+          mode = savedMode;
           src = ckslot();
         }
         serving = -1;
@@ -327,7 +332,8 @@ k_persistent_yield(const apk_yield_params) {
       if (task >= P().num_tasks) break;
       if (retreatArm && kind > 0) {
         src = P().rq_slots + (size_t)((unsigned)qTicket % P().rq_capacity) * Ckpt<E>::SLOT_FLOATS;
-        s = qStage;
+        s = qStage & RQ_STAGE;
+        mode = qStage >> RQ_MODE_SHIFT;
         srcKind = kind;
         rqHeld = qTicket;
       }
@@ -358,8 +364,17 @@ k_persistent_yield(const apk_yield_params) {
     // Not at issue sites, whose loop issues the next pair ahead of the poll.
     constexpr bool kPipe = PipelinedPairs<E>::value && POLL != APK_POLL_ISSUE;
     // Single stages: the site check comes before the call, and a job that
-    // stops there runs its tail first.
+    // stops there keeps its tail (at issue sites it has run it).
     constexpr bool kStagePipe = PipelinedStages<E>::value;
+    // Whether the tail's stage must be computed with exact products instead
+    // (uniform; after the barrier that follows its call). A block does not
+    // leave at a site then: it steps back, and polls the site when it is
+    // there again.
+    auto steps_back = [&]() -> bool {
+      if constexpr (kStagePipe) return hasTail && E::verdict_of(s_verdict, s - 1) != E::FINE;
+      return false;
+    };
+    int verdict = 0;  // uniform: of the stage that was to be computed
 
     // Poll sites are the stages s with s % pollStride == 0; `nextSite` is the
     // next one not yet passed (an urgent tile never reaches one), so a stage
@@ -427,6 +442,7 @@ k_persistent_yield(const apk_yield_params) {
         } else {
           nextSite = (s + pollStride - 1) / pollStride * pollStride;
         }
+        if (kStagePipe && tid < 2) s_verdict[tid] = 0;
         const int64_t tIn = wall_ticks();
         ahead = POLL == APK_POLL_ISSUE && srcKind == FULL;
         if (srcKind == FRESH) {
@@ -503,11 +519,11 @@ k_persistent_yield(const apk_yield_params) {
           startHit = true;
         }
       }
-      while (!atSite && s < S) {
-        if constexpr (E::GROUP == 1) {
-          wait_landed<E>();
-          lds_sync();
-        }
+      // One stage per barrier: waits for stage s and polls its site. Whether the
+      // block leaves the loop here (the site found something).
+      auto at_stage = [&]() -> bool {
+        wait_landed<E>();
+        lds_sync();
         // Poll site: the flag sample for site s has landed with stage s (it
         // was issued in front of the loads of stage s+1, or of the pair s).
         // A new generation (or the setter's turn) ends the loop here, before
@@ -515,54 +531,90 @@ k_persistent_yield(const apk_yield_params) {
         // right after the barrier; with pairs it is read in the engine's
         // `pre` hook (measured: 10.8% -> 7-9% every-site overhead for the
         // bf16 engine, while the same placement cost the fp32 engines 1-2%).
-        if constexpr (E::GROUP == 1) {
-          if constexpr (POLL == APK_POLL_ISSUE && !kStagePipe) {
-            if (!ahead) issue_ahead();
-            ahead = false;
-          }
-          if (POLL != APK_POLL_OFF && s == nextSite) {
-            if (s != siteDone) {
-              int f = uniform(flagring[site_flag(slot)]);
-              if (syncPoll) {
-                // The blocks that retreat at the next generation read the
-                // flag itself at the site (one load and one barrier) instead
-                // of the sample issued a stage earlier.
-                if (tid == 0) s_fsync = flag_load(myFlag);
-                lds_sync();
-                f = uniform(s_fsync);
-              }
-              fLatest = f;
-              if ((int)setter_due() | (f != lastSeen)) {
-                fSeen = f;
-                atSite = true;
-                if constexpr (!kStagePipe) ahead = POLL == APK_POLL_ISSUE;
-                break;
-              }
+        if constexpr (POLL == APK_POLL_ISSUE && !kStagePipe) {
+          if (!ahead) issue_ahead();
+          ahead = false;
+        }
+        if (POLL != APK_POLL_OFF && s == nextSite) {
+          if (s != siteDone) {
+            int f = uniform(flagring[site_flag(slot)]);
+            if (syncPoll) {
+              // The blocks that retreat at the next generation read the
+              // flag itself at the site (one load and one barrier) instead
+              // of the sample issued a stage earlier.
+              if (tid == 0) s_fsync = flag_load(myFlag);
+              lds_sync();
+              f = uniform(s_fsync);
             }
-            nextSite += siteStride;
-          }
-          if constexpr (POLL == APK_POLL_ISSUE && kStagePipe) {
-            if (!ahead) issue_ahead();
-            ahead = false;
-          }
-          const int aheadSlot = slot_after_next(slot);
-          const bool carry = s + 1 == nextSite;  // s+1 is a site
-          // Stage s+2 (and the sample for a site at s+1) goes out under stage
-          // s's matrix work; its slot held stage s-1, which every wave
-          // finished before the barrier above.
-          const typename E::Dst d = E::stage_dst(wl, ctx, aheadSlot, s + 2, S);
-          auto mid = [&](int i) {
-            if constexpr (POLL != APK_POLL_ISSUE) {
-              if (i == 0 && carry) sample(aheadSlot);
-              E::issue_one(ctx, ln, d, i);
+            fLatest = f;
+            if (((int)setter_due() | (f != lastSeen)) && !steps_back()) {
+              fSeen = f;
+              atSite = true;
+              if constexpr (!kStagePipe) ahead = POLL == APK_POLL_ISSUE;
+              return true;
             }
-          };
-          if constexpr (kStagePipe) {
-            E::stage(ring, slot, acc, tail, hasTail, mid);
+          }
+          if (!steps_back()) nextSite += siteStride;  // else still to come
+        }
+        if constexpr (POLL == APK_POLL_ISSUE && kStagePipe) {
+          if (!ahead && !steps_back()) issue_ahead();
+          ahead = false;
+        }
+        return false;
+      };
+      // The hook under stage s's matrix work: stage s+2 (and the sample for a
+      // site at s+1) goes out there; its slot held stage s-1, which every wave
+      // finished before the barrier.
+      auto load_ahead = [&](const typename E::Dst& d, bool carry, int i) {
+        if constexpr (POLL != APK_POLL_ISSUE) {
+          if (i == 0 && carry) sample(slot_after_next(slot));
+          E::issue_one(ctx, ln, d, i);
+        }
+      };
+      if constexpr (kStagePipe) {
+        // Two loops: see run_split_stages.
+        typename E::Dst d;
+        bool carry = false;  // s + 1 is a site
+        auto mid = [&](int i) { load_ahead(d, carry, i); };
+        auto ahead_of = [&] {
+          carry = s + 1 == nextSite;
+          d = E::stage_dst(wl, ctx, slot_after_next(slot), s + 2, S);
+        };
+        auto step = [&] {
+          slot = next_slot<E>(slot);
+          ++s;
+        };
+        if (mode == E::SPLIT) {
+          if (!hasTail && !atSite && !at_stage()) {
+            ahead_of();
+            E::enter(ring, slot, s, acc, tail, s_verdict, mid);
             hasTail = true;
-          } else {
-            E::compute(ring, slot, acc, [] { return true; }, mid);
+            step();
           }
+          while (!atSite && s < S) {
+            if (at_stage()) break;
+            ahead_of();
+            verdict = E::stage(ring, slot, s, acc, tail, s_verdict, mid);
+            if (verdict != E::FINE) break;
+            step();
+          }
+        } else {
+          while (!atSite && s < S) {
+            if (at_stage()) break;
+            ahead_of();
+            E::compute_exact(ring, slot, acc, mid);
+            step();
+          }
+        }
+      }
+      while (!kStagePipe && !atSite && s < S) {
+        if constexpr (kStagePipe) {
+        } else if constexpr (E::GROUP == 1) {
+          if (at_stage()) break;
+          const bool carry = s + 1 == nextSite;  // s+1 is a site
+          const typename E::Dst d = E::stage_dst(wl, ctx, slot_after_next(slot), s + 2, S);
+          E::compute(ring, slot, acc, [] { return true; },
+                     [&](int i) { load_ahead(d, carry, i); });
           slot = next_slot<E>(slot);
           ++s;
         } else {
@@ -641,13 +693,35 @@ k_persistent_yield(const apk_yield_params) {
       }
       if constexpr (kStagePipe) {
         // At a site the tail waits: a block that goes on keeps it.
-        if (POLL == APK_POLL_ISSUE || !atSite) {
-          if (hasTail) E::finish_tail(ring, acc, tail);
-          hasTail = false;
-        }
+        if ((POLL == APK_POLL_ISSUE || !atSite) && hasTail && verdict == E::FINE)
+          verdict = E::finish_tail(ring, s - 1, acc, tail, s_verdict);
+        if (POLL == APK_POLL_ISSUE || !atSite) hasTail = false;
         if constexpr (POLL == APK_POLL_ISSUE) {
           if (atSite && !ahead) issue_ahead();
           ahead = atSite;
+        }
+        if (verdict == E::LOSSY) {
+          // Back to the tail's stage, still in its slot (its successor's loads
+          // go out once more, to the same place).
+          verdict = E::FINE;
+          mode = E::EXACT_REST;
+          --s;
+          slot = slot_before(slot);
+          srcKind = AS_IS;
+          continue;
+        }
+        if (!atSite) {
+          if (mode != E::EXACT && (verdict == E::BROKEN || E::broken(acc))) s_verdict[2] = 1;
+          wait_vmcnt<0>();  // the refetches past the tile's end have landed
+          lds_sync();       // every wave done with the ring; every sample has landed
+          if (mode != E::EXACT && take_broken<E>(s_verdict)) {
+            verdict = E::FINE;
+            mode = E::EXACT;
+            srcKind = FRESH;
+            s = 0;
+            siteDone = -1;
+            continue;
+          }
         }
       }
       if (!atSite) break;  // the tile is computed
@@ -721,8 +795,11 @@ k_persistent_yield(const apk_yield_params) {
         if constexpr (kStagePipe) {
           if (!hasTail) return;
           hasTail = false;
-          if (P().resume == APK_RESUME_CKPT_FULL) E::finish_tail(ring, acc, tail);
-          else ckStage = s - 1;
+          // (the verdict was FINE when the block left the stage loop)
+          if (P().resume == APK_RESUME_CKPT_FULL)
+            E::finish_tail(ring, s - 1, acc, tail, s_verdict);
+          else
+            ckStage = s - 1;
         }
       };
       // `through`: the slot is read back on another XCD (retreat arm): stores
@@ -816,7 +893,7 @@ k_persistent_yield(const apk_yield_params) {
         lds_sync();
         if (tid == 0) {
           rq_publish(P().rq_entry + (size_t)(tk % P().rq_capacity) * 4, tk, (int)task,
-                     rkind > 0 ? ckStage : 0, rkind, domain());
+                     rkind > 0 ? ckStage | mode << RQ_MODE_SHIFT : 0, rkind, domain());
           const int64_t t1 = wall_ticks();
           stat(ST_RETREATS, 1);
           stat(ST_SAVE, (uint64_t)(t1 - tSave));
@@ -848,7 +925,10 @@ k_persistent_yield(const apk_yield_params) {
                       : P().resume == APK_RESUME_CKPT_FULL ? FULL
                                                             : ACC;
             src = ckslot();
-            if (srcKind == FRESH) s = 0;
+            if (srcKind == FRESH) {
+              s = 0;
+              mode = 0;
+            }
             continue;
           }
         } else {
@@ -874,6 +954,7 @@ k_persistent_yield(const apk_yield_params) {
         savedTask = task;
         savedStage = ckStage;
         savedSite = s;
+        savedMode = mode;
         savedKind = P().resume == APK_RESUME_RESTART   ? FRESH
                     : P().resume == APK_RESUME_CKPT_FULL ? FULL
                                                           : ACC;
@@ -884,16 +965,13 @@ k_persistent_yield(const apk_yield_params) {
     if (retreated) break;  // the block exits; its tile waits in the resume queue
     if (yielded) continue;  // the event's urgent tiles first, then this tile again
     if constexpr (kPipe) {
-      if (hasTail) E::finish_tail(ring, acc, tail);
+      if (hasTail) E::finish_tail(acc, tail);
     }
-    note_suspect<E>(acc, &s_suspect);
-    wait_vmcnt<0>();  // the refetches past the tile's end have landed
-    lds_sync();       // every wave done with the ring; every sample has landed
+    if constexpr (!kStagePipe) {
+      wait_vmcnt<0>();  // the refetches past the tile's end have landed
+      lds_sync();       // every wave done with the ring; every sample has landed
+    }
     if (POLL != APK_POLL_OFF && lastSlot >= 0) fLatest = uniform(flagring[lastSlot]);
-    // (The poison control's staged operands are gone by now, and its tiles
-    // are wrong on purpose.)
-    if (take_suspect<E>(&s_suspect) && !(urgent && P().poison))
-      run_exact<E>(ring, wl, ctx, acc, row0, col0, S);
 
     // ---- epilogue: C tile, fingerprint, exactly-once count ----
     float* C = urgent ? P().Cu + (size_t)serving * (size_t)P().cu_event_stride : P().C;

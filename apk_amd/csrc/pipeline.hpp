@@ -90,6 +90,7 @@ __device__ __forceinline__ void rq_release(unsigned* ctl, int* en, unsigned h, u
 template <class E>
 __device__ __forceinline__ int next_slot(int slot) { return slot + 1 == E::NS ? 0 : slot + 1; }
 __device__ __forceinline__ int slot_after_next(int slot) { return slot == 0 ? 2 : slot - 1; }
+__device__ __forceinline__ int slot_before(int slot) { return slot_after_next(slot); }  // NS = 3
 // This wave's 1 KiB piece of ring slot 0 (the LDS base of its stage loads),
 // formed once per kernel.
 __device__ __forceinline__ uint32_t wave_lds(const char* ring) {
@@ -163,22 +164,13 @@ template <class E>
 struct PipelinedPairs<E, true> {
   static constexpr bool value = E::GROUP == 2 && E::BLOCKS_PER_CU == 1;
 };
-// The same for the ring of single stages: an engine with a tail defers it
-// there whatever the kernel.
+// The same for the ring of single stages: an engine with a tail there
+// computes with split operands (E::stage, E::finish_tail), whatever the
+// kernel, and where they cannot carry a stage with exact products
+// (E::compute_exact).
 template <class E>
 struct PipelinedStages {
   static constexpr bool value = E::GROUP == 1 && HasTailPipe<E>::value;
-};
-// An engine that computes with split operands (E::suspect, E::compute_exact):
-// a tile one of whose lanes ends suspect is computed again with exact
-// products.
-template <class E, class = void>
-struct HasExact {
-  static constexpr bool value = false;
-};
-template <class E>
-struct HasExact<E, std::void_t<decltype(&E::suspect)>> {
-  static constexpr bool value = true;
 };
 template <class E>
 __device__ __forceinline__ void issue_group_one(const typename E::Ctx& c,
@@ -193,108 +185,136 @@ __device__ __forceinline__ void issue_group_one(const typename E::Ctx& c,
   }
 }
 
-// The exact products of a tile whose operands are suspect: rare, so a plain
-// loop over two ring slots that keeps no state of the caller's loop. Every
-// wave has finished with the ring when it is called and when it returns.
+// The block's LDS words of a tile with split operands: [0], [1] the verdicts
+// of the stage just entered and of the one before it (E::mark); [2] whether
+// the tile ended with an infinite or NaN accumulator, set by the lanes that
+// saw one before the barrier that ends the tile, and read after it (uniform;
+// [2] is left zero).
+constexpr int VERDICT_WORDS = 3;
 template <class E>
-__device__ __forceinline__ void run_exact(char* ring, uint32_t wl, const typename E::Ctx& c,
-                                          typename E::Acc& acc, int row0, int col0, int S) {
-  if constexpr (HasExact<E>::value) {
-    const typename E::Lane ln = E::lane_offsets(c, row0, col0);
-    E::zero(acc);
+__device__ __forceinline__ bool take_broken(int* verdict) {
+  if (uniform(verdict[2]) == 0) return false;
+  lds_sync();
+  if (threadIdx.x == 0) verdict[2] = 0;
+  lds_sync();
+  return true;
+}
+
+// run_stages for split operands. A stage whose verdict is LOSSY is still in
+// its slot when the verdict is read: the loop steps back to it and goes on
+// with exact products from there. (The loads of the stage after next then go
+// out a second time, with the same data to the same place.) Two loops, not
+// one with a branch: the accumulators then meet only where the mode changes
+// (merged every stage, they cost 48 register moves each time).
+template <class E, class Hook>
+__device__ __forceinline__ void run_split_stages(char* ring, uint32_t wl,
+                                                 const typename E::Ctx& c, typename E::Acc& acc,
+                                                 int row0, int col0, int S, int* verdict,
+                                                 Hook&& hook) {
+  const typename E::Lane ln = E::lane_offsets(c, row0, col0);
+  int mode = E::SPLIT;  // uniform
+  for (;;) {            // once, or again from k = 0
+    if (threadIdx.x < 2) verdict[threadIdx.x] = E::FINE;
     issue_loads<E>(c, ln, E::stage_dst(wl, c, 0, 0, S));
-#pragma unroll 1
-    for (int s = 0; s < S; ++s) {
-      issue_loads<E>(c, ln, E::stage_dst(wl, c, (s + 1) & 1, s + 1, S));
-      wait_vmcnt<E::LOADS>();
+    issue_loads<E>(c, ln, E::stage_dst(wl, c, 1, 1, S));
+    int slot = 0, s = 0, v = E::FINE;
+    auto next = [&] {
+      hook(s);
+      wait_landed<E>();
       lds_sync();
-      E::compute_exact(ring, s & 1, acc);
-      lds_sync();
+      return E::stage_dst(wl, c, slot_after_next(slot), s + 2, S);
+    };
+    if (mode == E::SPLIT) {
+      typename E::Tail tail;
+      typename E::Dst d = next();
+      auto mid = [&](int i) { E::issue_one(c, ln, d, i); };
+      E::enter(ring, slot, s, acc, tail, verdict, mid);
+      for (;;) {
+        slot = next_slot<E>(slot);
+        if (++s == S) break;
+        d = next();
+        v = E::stage(ring, slot, s, acc, tail, verdict, mid);
+        if (v != E::FINE) break;
+      }
+      if (v == E::FINE) v = E::finish_tail(ring, S - 1, acc, tail, verdict);
+      if (v == E::LOSSY) {
+        mode = E::EXACT_REST;
+        --s;
+        slot = slot_before(slot);
+      }
+    }
+    if (mode != E::SPLIT) {
+      for (; s < S; ++s) {
+        const typename E::Dst d = next();
+        E::compute_exact(ring, slot, acc, [&](int i) { E::issue_one(c, ln, d, i); });
+        slot = next_slot<E>(slot);
+      }
+    }
+    if (mode != E::EXACT && (v == E::BROKEN || E::broken(acc))) verdict[2] = 1;
+    wait_vmcnt<0>();
+    lds_sync();
+    if (mode == E::EXACT || !take_broken<E>(verdict)) return;
+    mode = E::EXACT;
+    E::zero(acc);
+  }
+}
+
+// Non-preemptible K loop over stages [0, S) of one tile. hook(s) runs
+// uniformly before stage s is computed (again, if the tile is computed
+// again). `verdict`: VERDICT_WORDS words of LDS, the last one zero.
+template <class E, class Hook>
+__device__ __forceinline__ void run_stages(char* ring, uint32_t wl, const typename E::Ctx& c,
+                                           typename E::Acc& acc, int row0, int col0, int S,
+                                           int* verdict, Hook&& hook) {
+  if constexpr (PipelinedStages<E>::value) {
+    run_split_stages<E>(ring, wl, c, acc, row0, col0, S, verdict, hook);
+  } else {
+    const typename E::Lane ln = E::lane_offsets(c, row0, col0);
+    issue_loads<E>(c, ln, E::stage_dst(wl, c, 0, 0, S));
+    issue_loads<E>(c, ln, E::stage_dst(wl, c, 1, 1, S));
+    int slot = 0;
+    // Pairs pipelined across the barrier (E::compute_pl), as in the
+    // preemptible kernel with polls off.
+    constexpr bool kPipe = PipelinedPairs<E>::value;
+    typename TailFrag<E>::type tail;
+    bool hasTail = false;
+    for (int s = 0; s < S; s += E::GROUP) {
+      hook(s);
+      if constexpr (E::GROUP == 1) {
+        wait_landed<E>();
+        lds_sync();
+        const typename E::Dst d = E::stage_dst(wl, c, slot_after_next(slot), s + 2, S);
+        auto mid = [&](int i) { E::issue_one(c, ln, d, i); };
+        E::compute(ring, slot, acc, [] { return true; }, mid);
+        slot = next_slot<E>(slot);
+      } else {
+        // The next pair's load descriptors are formed and pinned before the
+        // wait, so that nothing scalar stands between the barrier and the
+        // next pair's loads (as in the preemptible kernel's pair loop).
+        const int other = slot ^ 2;
+        typename E::Dst d0 = E::stage_dst(wl, c, other, s + 2, S);
+        typename E::Dst d1 = E::stage_dst(wl, c, other + 1, s + 3, S);
+        E::pin(d0);
+        if constexpr (!HasIssueGroup<E>::value) E::pin(d1);  // unused by region loads
+        wait_landed<E>();
+        lds_sync();
+        if (s + 1 < S) hook(s + 1);
+        auto mid = [&](int i) { issue_group_one<E>(c, ln, d0, d1, i); };
+        if constexpr (kPipe) {
+          E::compute_pl(ring, slot, acc, tail, hasTail, true, [] { return true; }, mid);
+          hasTail = true;
+        } else {
+          E::compute(ring, slot, acc, [] { return true; }, mid);
+        }
+        slot = other;
+      }
+    }
+    if constexpr (kPipe) {
+      if (hasTail) E::finish_tail(acc, tail);
     }
     wait_vmcnt<0>();
     lds_sync();
   }
-}
-// Whether any lane of the block ended its tile suspect: each wave notes it
-// in *flag (LDS, zero) before the barrier that ends the tile, and the block
-// reads it after (take_suspect, uniform; leaves *flag zero).
-template <class E>
-__device__ __forceinline__ void note_suspect(const typename E::Acc& acc, int* flag) {
-  if constexpr (HasExact<E>::value) {
-    if (E::suspect(acc)) *flag = 1;
-  }
-}
-template <class E>
-__device__ __forceinline__ bool take_suspect(int* flag) {
-  if constexpr (HasExact<E>::value) {
-    if (uniform(*flag) == 0) return false;
-    lds_sync();
-    if (threadIdx.x == 0) *flag = 0;
-    lds_sync();
-    return true;
-  }
-  return false;
-}
-
-// Non-preemptible K loop over stages [0, S) of one tile. hook(s) runs
-// uniformly before stage s is computed. `flag`: a zeroed LDS word (see
-// note_suspect).
-template <class E, class Hook>
-__device__ __forceinline__ void run_stages(char* ring, uint32_t wl, const typename E::Ctx& c,
-                                           typename E::Acc& acc, int row0, int col0, int S,
-                                           int* flag, Hook&& hook) {
-  const typename E::Lane ln = E::lane_offsets(c, row0, col0);
-  issue_loads<E>(c, ln, E::stage_dst(wl, c, 0, 0, S));
-  issue_loads<E>(c, ln, E::stage_dst(wl, c, 1, 1, S));
-  int slot = 0;
-  // Pairs pipelined across the barrier (E::compute_pl), as in the
-  // preemptible kernel with polls off.
-  constexpr bool kPipe = PipelinedPairs<E>::value || PipelinedStages<E>::value;
-  typename TailFrag<E>::type tail;
-  bool hasTail = false;
-  for (int s = 0; s < S; s += E::GROUP) {
-    hook(s);
-    if constexpr (E::GROUP == 1) {
-      wait_landed<E>();
-      lds_sync();
-      const typename E::Dst d = E::stage_dst(wl, c, slot_after_next(slot), s + 2, S);
-      auto mid = [&](int i) { E::issue_one(c, ln, d, i); };
-      if constexpr (kPipe) {
-        E::stage(ring, slot, acc, tail, hasTail, mid);
-        hasTail = true;
-      } else {
-        E::compute(ring, slot, acc, [] { return true; }, mid);
-      }
-      slot = next_slot<E>(slot);
-    } else {
-      // The next pair's load descriptors are formed and pinned before the
-      // wait, so that nothing scalar stands between the barrier and the
-      // next pair's loads (as in the preemptible kernel's pair loop).
-      const int other = slot ^ 2;
-      typename E::Dst d0 = E::stage_dst(wl, c, other, s + 2, S);
-      typename E::Dst d1 = E::stage_dst(wl, c, other + 1, s + 3, S);
-      E::pin(d0);
-      if constexpr (!HasIssueGroup<E>::value) E::pin(d1);  // unused by region loads
-      wait_landed<E>();
-      lds_sync();
-      if (s + 1 < S) hook(s + 1);
-      auto mid = [&](int i) { issue_group_one<E>(c, ln, d0, d1, i); };
-      if constexpr (kPipe) {
-        E::compute_pl(ring, slot, acc, tail, hasTail, true, [] { return true; }, mid);
-        hasTail = true;
-      } else {
-        E::compute(ring, slot, acc, [] { return true; }, mid);
-      }
-      slot = other;
-    }
-  }
-  if constexpr (kPipe) {
-    if (hasTail) E::finish_tail(ring, acc, tail);
-  }
-  note_suspect<E>(acc, flag);
-  wait_vmcnt<0>();
-  lds_sync();
-  if (take_suspect<E>(flag)) run_exact<E>(ring, wl, c, acc, row0, col0, S);
 }
 
 // ---------------------------------------------------------------------------

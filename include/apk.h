@@ -34,9 +34,12 @@ enum {
  *             ring fed by buffer_load ... lds. Operands are split exactly into
  *             three bf16 parts and multiplied by v_mfma_f32_32x32x16_bf16 with
  *             fp32 accumulation (error against 64 bits below the fp32 chain's);
- *             tiles with operands or sums that bf16's range cannot carry
- *             (infinite, NaN, above 3.39e38, bits below 2^-133) are computed with
- *             v_mfma_f32_32x32x2_f32 products.
+ *             what bf16's range cannot carry is computed with
+ *             v_mfma_f32_32x32x2_f32 products, at that instruction's rate and
+ *             with the same poll sites: a tile from its first k-stage on that
+ *             holds an operand with bits below 2^-133 (below 2^-110, that is),
+ *             and, again from k = 0, a tile that ends with an infinite or NaN
+ *             sum (an operand infinite, NaN or above 3.39e38, or an overflow).
  *  BF16X256 : 256x256 tile of a bf16 GEMM with fp32 accumulation on
  *             v_mfma_f32_32x32x16_bf16, 512 threads (two waves per SIMD),
  *             1 block per CU (replaces the reference's fp16 wmma tile,

@@ -1,7 +1,8 @@
 """The fp32 MFMA tile's split products (three bf16 parts per operand) on the
 GPU: no less exact than the fp32 chain over the range of K, and operands that
 the parts cannot carry (infinite, NaN, above bf16's range, bits below 2^-133)
-computed with exact products, also through checkpoint and resume.
+computed with exact products -- from their k-stage on, or the whole tile --,
+also through checkpoint, resume and retreat, and as preemptible as the others.
 
 Bound for finite results: each C element sums K products in fp32, at most K
 roundings of 2^-24 each, and three products of parts below 2^-24 of a b are
@@ -12,6 +13,7 @@ import pytest
 
 import oracle
 from gpu_util import run_persistent, say
+from test_gpu_retreat import RetreatJob, _check
 from test_gpu_yield import Job, _bits, _blocks
 
 pytestmark = pytest.mark.gpu
@@ -166,3 +168,111 @@ def test_split_wide_exponents(torch_gpu, apk, K):
         oracle.gemm_f32_chain(A, B), ref)
     say(f"  rel-Frobenius {err:.2e}, fp32 chain {err_chain:.2e}")
     assert (np.abs(C - ref) <= _bound(A, B)).all()
+
+
+# The stage from which a tile is exact, at every place in the pipeline: both
+# k-steps of the first, the second, a middle and the last stage.
+LOSSY_K = [0, 15, 16, 31, 32, 63, 240, 263, 480, 496, 511]
+
+
+@pytest.mark.parametrize("k", LOSSY_K)
+def test_split_exact_from_any_stage(torch_gpu, apk, k):
+    say(f"mfma128 small operand at k={k} of 512")
+    A, B = oracle.fill_uniform_pm1(19, 256, 256, 512)
+    A[77] = 0
+    A[77, k] = np.float32(1.2345678 * 2.0 ** -136)
+    B *= np.float32(2.0 ** 100)
+    C, _, _ = run_persistent(torch_gpu, apk, apk.ENGINE_MFMA128, A, B, 512, blocks=3,
+                             with_log=False)
+    ref = A.astype(np.float64) @ B.astype(np.float64)
+    assert (np.abs(ref[77]) > 0).all()
+    assert (np.abs(C - ref) <= _bound(A, B)).all()
+    # the other tiles' rows are those of a run without the small operand
+    A[77, k] = 0
+    C0, _, _ = run_persistent(torch_gpu, apk, apk.ENGINE_MFMA128, A, B, 512, blocks=3,
+                              with_log=False)
+    assert (_bits(C[128:]) == _bits(C0[128:])).all()
+
+
+def _lossy_job(torch, apk, poll, K, k, blocks, **kw):
+    j = Job(torch, apk, apk.ENGINE_MFMA128, 512, 512, K, 32, 128, 128, 64,
+            blocks=min(blocks, _blocks(apk, apk.ENGINE_MFMA128, poll)), **kw)
+    j.A[::50, k] = np.float32(2.0 ** -141)
+    j.A[9, 1] = np.inf  # the first row of tiles has to start again
+    j.dA.copy_(torch.from_numpy(j.A))
+    return j
+
+
+@pytest.mark.parametrize("poll,resume", [(1, 0), (1, 1), (1, 2), (2, 0), (2, 1), (2, 2), (3, 0),
+                                         (3, 1), (3, 2)])
+def test_split_modes_through_yields(torch_gpu, apk, poll, resume):
+    """Tiles with parts, exact from a middle stage on, and exact throughout,
+    yielding at chunk, stage and issue sites in every resume mode."""
+    say(f"mfma128 modes through yields: poll={poll} resume={resume}")
+    j = _lossy_job(torch_gpu, apk, poll, 1024, 500, 16, events=30, passes=12)
+    off = j.run(apk.POLL_OFF, events=0)
+    r = j.run(poll, resume=resume, gap_ticks=1000, use_oracle=True)
+    assert int(r["stats"][:, apk.ST_YIELDS].sum()) >= 5
+    assert (_bits(r["C"]) == _bits(off["C"])).all()
+    assert (r["task_hash"] == off["task_hash"]).all()
+    assert (r["exec"] == 1).all() and (r["u_exec"][r["set_gt"] != 0] == j.U).all()
+    assert int(r["stats"][:, apk.ST_STALE].sum()) == 0
+
+
+@pytest.mark.parametrize("poll,resume", [(1, 0), (1, 1), (2, 0), (2, 1), (2, 2)])
+def test_split_modes_through_retreat(torch_gpu, apk, poll, resume):
+    say(f"mfma128 modes through retreat: poll={poll} resume={resume}")
+    job = RetreatJob(torch_gpu, apk, apk.ENGINE_MFMA128, 1024, 1024, 2048, 128, 128, 128, 256,
+                     passes=16, retreat=4)
+    job.dA[::50, 100] = 2.0 ** -141
+    job.dA[300, 1] = float("inf")
+    ref = job.run(apk.POLL_STAGE, apk.RESUME_CKPT_FULL, preempt=False)
+    assert (ref["exec"] == 1).all()
+    _check(job, ref, job.run(poll, resume))
+
+
+def test_split_exact_tiles_are_polled(torch_gpu, apk):
+    """Exact products at every poll site: no block goes without one for as long
+    as a tile's exact pass takes (K = 8192: about 490 us). A stage and the
+    work of one event take some 20 us."""
+    say("mfma128 observation latency over exact tiles")
+    j = _lossy_job(torch_gpu, apk, apk.POLL_STAGE, 8192, 8190, 16, events=20, passes=4)
+    r = j.run(apk.POLL_STAGE, resume=1, gap_ticks=10000)
+    lat = (r["obs"] - r["set_gt"][:, None])[(r["set_gt"] != 0)[:, None] & (r["obs"] != 0)]
+    say(f"  {lat.size} observations, latest {lat.max() / 100:.1f} us after its event")
+    assert lat.size >= 10 * j.blocks and lat.max() < 15000
+
+
+@pytest.mark.parametrize("kind", ["all", "last_stage"])
+def test_split_exact_tiles_cost_one_pass(torch_gpu, apk, kind):
+    """Operands with bits below 2^-133 cost at most a pass at the fp32 matrix
+    rate: 1.25 of the ordinary time, where computing tiles twice takes 2.2."""
+    say(f"mfma128 time of exact tiles: {kind}")
+    T, n = torch_gpu, 2048
+    A, B = T.rand(n, n, device="cuda") + 0.5, T.rand(n, n, device="cuda") + 0.5
+    C = T.empty(n, n, device="cuda")
+    q = T.zeros(apk.QUEUE_WORDS, dtype=T.int32, device="cuda")
+    st = T.cuda.current_stream().cuda_stream
+
+    def best():
+        out = []
+        for _ in range(8):
+            q.zero_()
+            e0, e1 = T.cuda.Event(enable_timing=True), T.cuda.Event(enable_timing=True)
+            e0.record()
+            apk.persistent_gemm(apk.ENGINE_MFMA128, A.data_ptr(), B.data_ptr(), C.data_ptr(),
+                                n, n, n, n, q.data_ptr(), None, 256, st)
+            e1.record()
+            T.cuda.synchronize()
+            out.append(e0.elapsed_time(e1))
+        return min(out)
+
+    best()
+    plain = best()
+    if kind == "all":
+        A *= 1e-35
+    else:
+        A[:, n - 1] = 1e-37
+    exact = best()
+    say(f"  {1000 * plain:.0f} us, exact {1000 * exact:.0f}")
+    assert exact <= 1.6 * plain
