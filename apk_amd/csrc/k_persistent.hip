@@ -101,7 +101,13 @@ __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu
 // 100-112): one block per output tile, block b computing tile b over the
 // whole K, no queue; block 0 stamps the job's start at its first
 // instruction and every block raises the job's end once its tile is stored.
-template <class E>
+// A tile may be handed out in FM x FN parts of E's size: the parts of tile t
+// then go to the blocks of XCD t % 8, where the whole tile would run, so that
+// an XCD's L2 holds the same operand panels either way. (Dealt row by row, or
+// in runs per XCD, some shapes of 42 to 64 parts spilled an L2 that the whole
+// tiles fit, and ran at 0.64 to 0.77 of their speed with warm operands.)
+// Blocks past the last tile have nothing to do.
+template <class E, int FM, int FN>
 __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu(E::MIN_WAVES_PER_SIMD, E::WAVES_PER_SIMD)))
     k_urgent_tiles(const void* __restrict__ A, const void* __restrict__ B,
                    float* __restrict__ C, int M, int N, int K, long long* start_gt,
@@ -110,9 +116,16 @@ __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu
   __shared__ __attribute__((aligned(16))) char ring[E::LDS_BYTES];
   __shared__ int s_verdict[VERDICT_WORDS];
   if (threadIdx.x == 0) s_verdict[2] = 0;  // first read after a stage's barrier
-  const int tilesN = N / E::TN;
-  const int row0 = (int)(blockIdx.x / (unsigned)tilesN) * E::TM;
-  const int col0 = (int)(blockIdx.x % (unsigned)tilesN) * E::TN;
+  const unsigned tilesN = (unsigned)N / (E::TN * FN);
+  unsigned tile = blockIdx.x, part = 0;
+  if constexpr (FM * FN > 1) {
+    const unsigned i = blockIdx.x / APK_QUEUE_XCDS;
+    tile = i / (FM * FN) * APK_QUEUE_XCDS + blockIdx.x % APK_QUEUE_XCDS;
+    part = i % (FM * FN);
+    if (tile >= (unsigned)M / (E::TM * FM) * tilesN) return;
+  }
+  const int row0 = (int)(tile / tilesN * FM + part / FN) * E::TM;
+  const int col0 = (int)(tile % tilesN * FN + part % FN) * E::TN;
   const typename E::Ctx ctx = E::make_ctx(A, B, M, N, K);
   typename E::Acc acc;
   E::zero(acc);
@@ -198,10 +211,14 @@ static int scratch_of_current_device(unsigned** out) {
 // The tile an urgent job of few tiles is computed with: the latency of such a
 // job is that of one block's tile, so the bf16 tiles of several 128x128 parts
 // are handed to as many blocks instead (each tile's C is bit-identical, as
-// every output's sum has the same order): bf16x256 256^3 8.9 -> 4.1 us,
-// 512^3 13.2 -> 5.7, 1024x1024x4096 75 -> 42; bf16x256x128 512^3 8.7 -> 6.4,
-// 1024x1024x4096 71 -> 50. What bounds it: one wave per SIMD, whose operand
-// reads and MFMAs of a k-step follow the barrier of its load region.
+// every output's sum has the same order): bf16x256 256^3 8.9 -> 4.4 us,
+// 512^3 13.2 -> 5.8, 1024x1024x4096 75 -> 41; bf16x256x128 512^3 8.7 -> 6.6,
+// 1024x1024x4096 71 -> 49. What bounds it: one wave per SIMD, whose operand
+// reads and MFMAs of a k-step follow the barrier of its load region. Over 38
+// tile grids of 2 to 64 parts (odd ones among them) and K = 32..4096, against
+// the engine's own tile: bf16x256 1.3-2.7 times as fast with warm operands,
+// 1.4-1.7 with cold ones; bf16x256x128 1.2-1.5 with either (1.0-1.2 below K =
+// 128, where both are little more than a launch).
 // The line: at most two such blocks per dispatch domain, which is what one CU
 // holds of them. An urgent job that waits for the retreat arm's freed CUs, one
 // per domain, then still starts at once; larger jobs keep the engine's own
@@ -232,14 +249,15 @@ static int launch_urgent_tiles(const void* A, const void* B, float* C, int M, in
   static_assert(E::TM % U::TM == 0 && E::TN % U::TN == 0 &&
                     KAlign<E>::value == KAlign<U>::value && E::KS == U::KS,
                 "every shape that E takes is one of U's");
-  const long long parts = (long long)(M / U::TM) * (N / U::TN);
-  if (parts <= kUrgentParts) {
-    hipLaunchKernelGGL(k_urgent_tiles<U>, dim3((int)parts), dim3(U::THREADS), 0, st, A, B, C, M,
-                       N, K, start_gt, end_gt);
+  constexpr int FM = E::TM / U::TM, FN = E::TN / U::TN;
+  const int tiles = (M / E::TM) * (N / E::TN);
+  if (FM * FN > 1 && tiles <= kUrgentParts / (FM * FN)) {
+    const int rounds = (tiles + APK_QUEUE_XCDS - 1) / APK_QUEUE_XCDS;
+    hipLaunchKernelGGL((k_urgent_tiles<U, FM, FN>), dim3(rounds * APK_QUEUE_XCDS * FM * FN),
+                       dim3(U::THREADS), 0, st, A, B, C, M, N, K, start_gt, end_gt);
   } else {
-    const int tiles = (M / E::TM) * (N / E::TN);
-    hipLaunchKernelGGL(k_urgent_tiles<E>, dim3(tiles), dim3(E::THREADS), 0, st, A, B, C, M, N, K,
-                       start_gt, end_gt);
+    hipLaunchKernelGGL((k_urgent_tiles<E, 1, 1>), dim3(tiles), dim3(E::THREADS), 0, st, A, B, C,
+                       M, N, K, start_gt, end_gt);
   }
   APK_LAUNCHED();
   return APK_OK;

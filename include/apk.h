@@ -138,9 +138,9 @@ int apk_persistent_gemm(int engine, const void* A, const void* B, float* C,
  * per output tile, block b computing tile b (row-major tile order) over the
  * whole K, with no work queue (nothing to clear, nothing allocated). A job of
  * bf16x256 or bf16x256x128 tiles that makes at most 64 128x128 parts runs one
- * block per part instead, in row-major part order. Same
- * operands, layouts and per-element k order as apk_persistent_gemm, so C is
- * bit-identical to it. Optional outputs (device memory, may be NULL):
+ * block per part instead, a tile's parts on one XCD (and surplus blocks that
+ * return at once, up to the next 8 tiles). Same operands, layouts and
+ * per-element k order as apk_persistent_gemm, so C is bit-identical to it. Optional outputs (device memory, may be NULL):
  * *start_gt = wall-clock ticks at block 0's first instruction (the
  * reference's uStartGT); *end_gt raised (atomic max, unsigned) to the time
  * each block's tile is stored (the reference's uEndGT; the caller zeroes

@@ -70,7 +70,9 @@ def test_urgent_bf16_matches_persistent(torch_gpu, apk, name):
     ("bf16x256", 256, 256, 64), ("bf16x256", 256, 768, 192), ("bf16x256", 2048, 512, 128),
     ("bf16x256", 2304, 512, 128), ("bf16x256x128", 256, 128, 32),
     ("bf16x256x128", 512, 384, 160), ("bf16x256x128", 1024, 1024, 96),
-    ("bf16x256x128", 256, 4224, 96)])
+    ("bf16x256x128", 256, 4224, 96),
+    # tile counts that leave surplus blocks: 5 and 9 of 8 and 16, 21 of 24
+    ("bf16x256", 256, 1280, 64), ("bf16x256", 768, 768, 64), ("bf16x256x128", 768, 896, 96)])
 def test_urgent_bf16_parts(torch_gpu, apk, name, M, N, K):
     torch = torch_gpu
     eng = apk.ENGINES[name]
@@ -93,6 +95,38 @@ def test_urgent_bf16_parts(torch_gpu, apk, name, M, N, K):
     # most the result's
     assert oracle.rel_frobenius(C, ref) <= 2.0 ** -24 * K
     assert 0 < start <= end
+
+
+@pytest.mark.parametrize("M,N,K", [(768, 896, 1568), (512, 2048, 2080)])
+def test_urgent_bf16_parts_share_an_l2(torch_gpu, apk, M, N, K):
+    """Each part of a job has a CU of its own, so a job of many parts takes
+    about as long as one of two, as long as an XCD's L2 (4 MiB) holds what its
+    blocks read. It does where a tile's parts run on one XCD; dealt row by row
+    (in runs per XCD) the first (second) job took 2.1 times as long."""
+    torch, eng = torch_gpu, apk.ENGINES["bf16x256x128"]
+    say(f"urgent_gemm bf16x256x128 {M}x{N}x{K}: time against 256x128x{K}")
+    A = torch.randn(M, K, device="cuda").to(torch.bfloat16)
+    B = torch.randn(N, K, device="cuda").to(torch.bfloat16)
+    C = torch.empty(M, N, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+
+    def us(m, n):
+        best = []
+        for _ in range(8):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            for _ in range(20):
+                apk.urgent_gemm(eng, A.data_ptr(), B.data_ptr(), C.data_ptr(), m, n, K, None,
+                                None, st)
+            e1.record()
+            torch.cuda.synchronize()
+            best.append(50 * e0.elapsed_time(e1))
+        return min(best)
+
+    us(M, N)
+    many, two = us(M, N), us(256, 128)
+    say(f"  {many:.1f} us, two parts {two:.1f}")
+    assert many <= 1.6 * two
 
 
 def test_urgent_rejects_bad_shape(torch_gpu, apk):
