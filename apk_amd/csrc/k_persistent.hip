@@ -22,7 +22,7 @@ template <class E>
 __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu(E::MIN_WAVES_PER_SIMD, E::WAVES_PER_SIMD)))
     k_persistent_gemm(const void* __restrict__ A, const void* __restrict__ B,
                       float* __restrict__ C, int M, int N, int K, int kChunk,
-                      unsigned* next_task, apk_tile_record* log) {
+                      unsigned* next_task, apk_tile_record* log, unsigned workers) {
   __shared__ __attribute__((aligned(16))) char ring[E::LDS_BYTES];
   __shared__ unsigned s_task;
   __shared__ proto::QueueCursor s_cur;  // thread 0's place in the queue
@@ -30,9 +30,9 @@ __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu
 
   const int tilesN = N / E::TN;
   const unsigned numTasks = (unsigned)((M / E::TM) * tilesN);
-  // The launch owns its counters: every worker's first task is fixed.
-  const TaskQueue tq(next_task, M / E::TM, tilesN, numTasks, gridDim.x);
-  const int home = (int)xcc_id();
+  const TaskQueue tq(next_task, M / E::TM, tilesN, numTasks);
+  // Blocks are dealt to the XCDs in turn, so blocks of one list share an L2.
+  const int home = tq.home_of((int)(blockIdx.x % APK_QUEUE_XCDS));
   const int nChunks = K / kChunk;
   const int spc = kChunk / E::KS;  // k-stages per chunk
   const typename E::Ctx ctx = E::make_ctx(A, B, M, N, K);
@@ -40,14 +40,13 @@ __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu
   if (threadIdx.x == 0) {
     s_verdict[2] = 0;
     s_cur = proto::QueueCursor{0, 0, 0, 0, 0};
-    tq.start(s_cur, blockIdx.x);
   }
 
   for (;;) {
     // Reconverge before the thread-0 pop (no thread-0 region of the previous
     // iteration may be threaded into this one across the back-edge).
     lds_sync();
-    if (threadIdx.x == 0) s_task = tq.pop(home, s_cur);
+    if (threadIdx.x == 0) s_task = tq.pop(home, s_cur, 1, gridDim.x);
     __syncthreads();
     const unsigned task = uniform(s_task);
     __syncthreads();  // every thread has read s_task before it is rewritten
@@ -88,12 +87,12 @@ __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu
       rec[nChunks - 1].block = (int)blockIdx.x;
     }
   }
-  // The counters end as if every worker had taken its first task from them
-  // and failed once on every list: one block adds that for all, with one
-  // request, after the last task is handed out.
+  // A drained list's counter ends at its length and one request more of every
+  // worker at least, by which a caller can tell it from one whose last tasks
+  // still run. Workers no longer make that request, so one block makes it for
+  // all, after the last task is handed out.
   if (blockIdx.x == 0 && threadIdx.x < APK_QUEUE_XCDS && tq.list_total((int)threadIdx.x) > 0)
-    __hip_atomic_fetch_add(&next_task[threadIdx.x],
-                           gridDim.x + tq.list_first((int)threadIdx.x), __ATOMIC_RELAXED,
+    __hip_atomic_fetch_add(&next_task[threadIdx.x], workers, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -168,8 +167,12 @@ static int launch_persistent_gemm(const void* A, const void* B, float* C,
   const int rc = validate_persistent_gemm<E>(A, B, C, M, N, K, kChunk, blocks);
   if (rc != APK_OK) return rc;
   APK_REQUIRE(next != nullptr, "persistent_gemm: next_task is NULL");
-  hipLaunchKernelGGL(k_persistent_gemm<E>, dim3(blocks), dim3(E::THREADS), 0, st,
-                     A, B, C, M, N, K, kChunk, next, log);
+  // A worker beyond the number of tiles can find nothing to do: not launched, it
+  // costs the queue neither its request nor its look at the counters.
+  const long long tiles = (long long)(M / E::TM) * (N / E::TN);
+  const int workers = blocks < tiles ? blocks : (int)tiles;
+  hipLaunchKernelGGL(k_persistent_gemm<E>, dim3(workers), dim3(E::THREADS), 0, st,
+                     A, B, C, M, N, K, kChunk, next, log, (unsigned)blocks);
   APK_LAUNCHED();
   return APK_OK;
 }

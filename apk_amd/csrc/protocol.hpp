@@ -51,16 +51,17 @@ namespace proto {
 //  - a list it has found exhausted it never tries again, and on finding one
 //    it reads all eight counters at once instead of trying the other lists
 //    one atomic at a time (with 1024 workers those 8 failing atomics each
-//    were most of the 111 us of a 221-tile GEMM; now 28 us);
+//    were most of the 111 us of a 221-tile GEMM); it reads them too before
+//    it asks a list that has fewer positions left than workers;
 //  - short tasks are taken several at a time (`batch`), fewer as the list
-//    runs out;
-//  - `statics` > 0 (a launch that owns its counters): worker b starts with
-//    position b / 8 of list b % 8, no atomic at all, and the counters hand
-//    out the positions after those.
+//    runs out.
+// Every task goes through the counters, so whatever launches share them, now
+// or one after the other, and however few of a launch's workers run, each
+// task is handed out once and the workers that do run take them all.
 constexpr unsigned TQ_NONE = 0xffffffffu;
 // One worker's place in the queue: positions [next, end) of `list` are its
-// own; bit q of `dead` marks list q exhausted; `seen` is the last index its
-// own list's counter gave it. All zero at the start.
+// own; bit q of `dead` marks list q exhausted; `seen` is one more than the
+// last index its own list's counter gave it. All zero at the start.
 struct QueueCursor {
   unsigned next, end, list, dead, seen;
 };
@@ -69,11 +70,11 @@ struct TaskQueue {
   static constexpr int GM = 4;
   unsigned* ctr;
   int tilesM, tilesN, T;
-  unsigned numTasks, passes, statics;
+  unsigned numTasks, passes;
 
-  APK_PROTO_FN TaskQueue(unsigned* c, int tm, int tn, unsigned n, unsigned st = 0)
+  APK_PROTO_FN TaskQueue(unsigned* c, int tm, int tn, unsigned n)
       : ctr(c), tilesM(tm), tilesN(tn), T(tm * tn), numTasks(n),
-        passes((n + (unsigned)(tm * tn) - 1) / (unsigned)(tm * tn)), statics(st) {}
+        passes((n + (unsigned)(tm * tn) - 1) / (unsigned)(tm * tn)) {}
 
   APK_PROTO_FN int grouped(int i) const {
     const int band = i / (GM * tilesN);
@@ -85,27 +86,28 @@ struct TaskQueue {
   APK_PROTO_FN int list_begin(int q) const {
     return (int)(((long long)q * T) / APK_QUEUE_XCDS);
   }
-  // Positions of list q over all passes, and how many of them are the
-  // workers' first tasks.
+  // The list that workers x, x + 8, ... of a grid call their own: T % 8 lists
+  // hold one position more than the others, and go to the first T % 8 values
+  // of x. Of T workers, one for each position, as many then start on a list as
+  // it has positions, and none has to steal.
+  APK_PROTO_FN int home_of(int x) const {
+    const int rest = T % APK_QUEUE_XCDS;
+    int y = x < rest ? x : x - rest;
+    for (int q = 0; q < APK_QUEUE_XCDS; ++q) {
+      const bool longer = (q + 1) * rest / APK_QUEUE_XCDS != q * rest / APK_QUEUE_XCDS;
+      if (longer == (x < rest) && y-- == 0) return q;
+    }
+    return x;  // not reached
+  }
+  // Positions of list q over all passes.
   APK_PROTO_FN unsigned list_total(int q) const {
     return (unsigned)(list_begin(q + 1) - list_begin(q)) * passes;
-  }
-  APK_PROTO_FN unsigned list_first(int q) const {
-    const unsigned w = (statics + APK_QUEUE_XCDS - 1 - (unsigned)q) / APK_QUEUE_XCDS;
-    const unsigned total = list_total(q);
-    return w < total ? w : total;
   }
   // Whether any position is still to be handed out.
   APK_PROTO_FN bool any_left() const {
     for (int q = 0; q < APK_QUEUE_XCDS; ++q)
-      if (P::load(&ctr[q]) < list_total(q) - list_first(q)) return true;
+      if (P::load(&ctr[q]) < list_total(q)) return true;
     return false;
-  }
-  // Worker b's first task (statics > b): nothing if its list is shorter.
-  APK_PROTO_FN void start(QueueCursor& c, unsigned b) const {
-    c.list = b % APK_QUEUE_XCDS;
-    c.next = b / APK_QUEUE_XCDS;
-    c.end = c.next < list_first((int)c.list) ? c.next + 1 : c.next;
   }
   // One caller per block. Returns the next task id, or TQ_NONE when every
   // list is exhausted. `batch` > 1: up to that many consecutive positions of
@@ -118,8 +120,18 @@ struct TaskQueue {
     cursor = c;
     return u;
   }
+  // Marks the lists that all the counters, read in one round trip, show
+  // exhausted. A counter only grows, so a list seen exhausted stays so.
+  APK_PROTO_FN void look(QueueCursor& c) const {
+    unsigned v[APK_QUEUE_XCDS];
+    for (int i = 0; i < APK_QUEUE_XCDS; ++i) v[i] = P::load(&ctr[i]);
+    for (int i = 0; i < APK_QUEUE_XCDS; ++i)
+      if (v[i] >= list_total(i)) c.dead |= 1u << i;
+  }
   APK_PROTO_FN unsigned pop_local(int home, QueueCursor& c, unsigned batch,
                                   unsigned workers) const {
+    const unsigned each = (workers + APK_QUEUE_XCDS - 1) / APK_QUEUE_XCDS;  // of a list
+    bool looked = false;
     for (;;) {
       if (c.next < c.end) {
         const int b = list_begin((int)c.list);
@@ -135,28 +147,30 @@ struct TaskQueue {
         if (k == APK_QUEUE_XCDS) return TQ_NONE;
       }
       const int q = (home + k) & (APK_QUEUE_XCDS - 1);
-      const unsigned first = list_first(q), total = list_total(q) - first;
+      const unsigned total = list_total(q);
+      // Fewer positions left than workers, by the last index seen: the others
+      // have most likely taken them, so look before asking.
+      if (k == 0 && c.seen > 0 && !looked && total - c.seen <= each) {
+        looked = true;
+        look(c);
+        continue;
+      }
       unsigned take = 1;
       if (k == 0 && batch > 1) {
-        const unsigned each = (total - c.seen) / (workers + APK_QUEUE_XCDS - 1);
-        take = each < 1 ? 1 : each < batch ? each : batch;
+        const unsigned share = (total - c.seen) / (workers + APK_QUEUE_XCDS - 1);
+        take = share < 1 ? 1 : share < batch ? share : batch;
       }
       unsigned j = total;
       if (total > 0) j = P::fetch_add(&ctr[q], take);
       if (j < total) {
-        if (k == 0) c.seen = j;
+        if (k == 0) c.seen = j + 1;
         c.list = (unsigned)q;
-        c.next = first + j;
-        c.end = first + (total - j < take ? total : j + take);
+        c.next = j;
+        c.end = total - j < take ? total : j + take;
         continue;
       }
-      // Exhausted: look at all the counters in one round trip. A counter
-      // only grows, so a list seen exhausted stays so.
       c.dead |= 1u << q;
-      unsigned v[APK_QUEUE_XCDS];
-      for (int i = 0; i < APK_QUEUE_XCDS; ++i) v[i] = P::load(&ctr[i]);
-      for (int i = 0; i < APK_QUEUE_XCDS; ++i)
-        if (v[i] >= list_total(i) - list_first(i)) c.dead |= 1u << i;
+      look(c);
     }
   }
 };

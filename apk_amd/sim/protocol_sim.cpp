@@ -30,8 +30,7 @@
 // --rq-wait-us sets the ring's wait deadlines (the kernels' 20 ms by default).
 // --urgent-us: how long the urgent kernel holds the freed CUs before the
 // continuation starts (20 us by default).
-// --batch: tasks per pop; --statics 1: every block's first task is fixed (both
-// cooperative arm only).
+// --batch: tasks per pop (cooperative arm).
 // --bug plants one mistake, to show that the checks see it:
 //   publish-early   (retreat) publish the ticket before writing the slot
 //   resume-skip     resume one stage past the checkpointed stage
@@ -142,7 +141,6 @@ struct Config {
   int workNs = 2000, pollEvery = 1, resume = R_FULL, retreatN = 32, cap = 0, urgentTiles = 4;
   int domains = APK_RETREAT_DOMAINS;
   int batch = 1;         // tasks per pop (cooperative arm)
-  bool statics = false;  // fixed first tasks (cooperative arm)
   int64_t rqWaitTicks = proto::RQ_WAIT_TICKS;
   int64_t urgentNs = 20000;
   unsigned seed = 21;
@@ -230,12 +228,9 @@ struct Sim {
     if (c.retreat)
       mayRetreat = cont ? epoch > 0 && epoch < c.events
                         : __atomic_fetch_add(&regCount[dom], 1, __ATOMIC_RELAXED) < quota;
-    const bool fixedFirst = c.statics && !c.retreat;
-    proto::TaskQueue<HostPlat> tq(ctr.data(), c.tilesM, c.tilesN, numTasks,
-                                  fixedFirst ? (unsigned)c.blocks : 0u);
+    proto::TaskQueue<HostPlat> tq(ctr.data(), c.tilesM, c.tilesN, numTasks);
     const unsigned T = (unsigned)(c.tilesM * c.tilesN);
     proto::QueueCursor cursor{0, 0, 0, 0, 0};
-    if (fixedFirst) tq.start(cursor, (unsigned)bid);
     for (;;) {
       // ---- the next task: resume ring first (retreat arm), else the queue ----
       unsigned task = 0xffffffffu;
@@ -446,7 +441,6 @@ int main(int argc, char** argv) {
     else if (k == "--rq-wait-us") c.rqWaitTicks = (int64_t)(atof(v) * 100.0);
     else if (k == "--urgent-us") c.urgentNs = (int64_t)(atof(v) * 1000.0);
     else if (k == "--batch") c.batch = atoi(v);
-    else if (k == "--statics") c.statics = atoi(v) != 0;
     else if (k == "--bug") bug = v;
     else {
       fprintf(stderr, "unknown option %s\n", k.c_str());

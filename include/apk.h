@@ -242,13 +242,13 @@ enum {
 };
 
 /* Work queue: every persistent kernel pops tasks from APK_QUEUE_WORDS
- * unsigned counters (zero at launch, and the launch's own until it ends; the
- * retreat arm's continuations join its first grid's). The tiles are split into
+ * unsigned counters, zero at launch. Launches of one job may share them (the
+ * retreat arm's continuations join its first grid's): each takes what the
+ * others have not. The tiles are split into
  * APK_QUEUE_XCDS lists, one per XCD, each a compact 2-D region of the tile
  * grid; a worker pops from its own XCD's list first (so concurrently running
  * tiles share A and B panels in that XCD's L2) and steals from the others
- * when it is empty. A worker of apk_persistent_gemm starts with a fixed task
- * (position b / 8 of list b % 8 for block b). Task u always computes tile u mod (tilesM * tilesN). */
+ * when it is empty. Task u always computes tile u mod (tilesM * tilesN). */
 #define APK_QUEUE_WORDS 16
 #define APK_QUEUE_XCDS 8
 /* Control words of the retreat arm's resume ring (apk_yield_params.rq_ctl). */

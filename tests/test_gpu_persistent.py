@@ -109,3 +109,40 @@ def test_cfg2_full_size_sampled_rows(torch_gpu, apk, cfg2_operands, kc):
         assert oracle.rel_frobenius(C[r:r + 1], ref) <= FROB_F32, r
     assert (recs["block"] >= 0).all()
     assert len(recs["block"]) == 32 * 32 * (4096 // kc)
+
+
+@pytest.mark.parametrize("name", ["valu64", "mfma128", "bf16x256", "bf16x256x128", "bf16x128"])
+def test_launches_share_a_queue(torch_gpu, apk, name):
+    """Every tile goes through the caller's counters: launches that share them
+    compute each tile once, and one that finds them drained computes nothing."""
+    say(f"{name}: shared queue counters")
+    T, eng = torch_gpu, apk.ENGINES[name]
+    g = apk.geometry(eng)
+    tm, tn, K = 3, 5, 64
+    M, N = tm * g.tile_m, tn * g.tile_n
+    kind = T.bfloat16 if g.elem_bytes == 2 else T.float32
+    A = T.rand(M, K, device="cuda").to(kind)
+    B = T.rand(N * K, device="cuda").to(kind)
+    q = T.zeros(apk.QUEUE_WORDS, dtype=T.int32, device="cuda")
+
+    def run(blocks):
+        """Which tiles a launch wrote."""
+        C = T.full((M, N), float("nan"), device="cuda")
+        apk.persistent_gemm(eng, A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, K,
+                            q.data_ptr(), None, blocks, T.cuda.current_stream().cuda_stream)
+        T.cuda.synchronize()
+        done = ~C.isnan().view(tm, g.tile_m, tn, g.tile_n)
+        whole = done.all(dim=3).all(dim=1)
+        assert (whole == done.any(dim=3).any(dim=1)).all()
+        return whole
+
+    assert run(64).all()
+    assert not run(64).any()  # drained
+    # another launch has taken the first position of every list with two
+    sizes = [(i + 1) * tm * tn // 8 - i * tm * tn // 8 for i in range(8)]
+    q.zero_()
+    q[:8] = T.tensor([1 if n == 2 else 0 for n in sizes], dtype=T.int32, device="cuda")
+    for blocks in (2, 64):  # few workers take all that is left; the next launch nothing
+        left = run(blocks)
+        want = tm * tn - sizes.count(2) if blocks == 2 else 0
+        assert int(left.sum()) == want

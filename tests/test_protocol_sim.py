@@ -198,7 +198,6 @@ def test_retreat_short_ring_waits(seed):
 
 
 @pytest.mark.parametrize("batch", [1, 3, 8])
-@pytest.mark.parametrize("statics", [0, 1])
 @pytest.mark.parametrize("blocks,tiles_m,tiles_n,passes", [
     (16, 1, 1, 1),    # one tile: seven empty lists
     (3, 3, 2, 1),     # fewer workers than lists, fewer tiles than lists
@@ -206,12 +205,12 @@ def test_retreat_short_ring_waits(seed):
     (16, 2, 4, 1),    # one position per list
     (16, 16, 16, 16), # batches shrink as the lists run out
 ])
-def test_queue_hands_out_every_task_once(batch, statics, blocks, tiles_m, tiles_n, passes):
-    """Several tasks per pop and fixed first tasks, over list lengths from
-    zero up: every task done exactly once."""
+def test_queue_hands_out_every_task_once(batch, blocks, tiles_m, tiles_n, passes):
+    """Several tasks per pop, over list lengths from zero up: every task done
+    exactly once."""
     rc, line, f = run("--arm", "coop", "--blocks", blocks, "--tiles-m", tiles_m, "--tiles-n",
                       tiles_n, "--passes", passes, "--stages", 2, "--work-ns", 200, "--events", 3,
-                      "--batch", batch, "--statics", statics, job=False)
+                      "--batch", batch, job=False)
     assert rc == 0 and line.startswith("PASS"), line
     assert f["dup"] == 0 and f["miss"] == 0, line
 
