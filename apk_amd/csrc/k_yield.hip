@@ -187,9 +187,7 @@ k_persistent_yield(const apk_yield_params) {
   // Whether the setter has something to do at this site (uniform; called
   // once per site, after a barrier).
   proto::SetterLook<DevPlat> look{s_due, 0};
-  auto setter_due = [&]() -> bool {
-    return isSetter && look.at_site(tid == 0, [&] { return wall_ticks() >= s_setter[2]; });
-  };
+  auto setter_due = [&]() -> bool { return isSetter && look.at_site(); };
 
   // Broadcast a value thread 0 computed (uniform afterwards).
   auto bcast = [&](unsigned v) -> unsigned {
@@ -390,6 +388,9 @@ k_persistent_yield(const apk_yield_params) {
       if (POLL != APK_POLL_OFF) {
         sample_flag<SYS>(flag_rsrc, flag_lds + 4u * (uint32_t)idx);
         lastSlot = idx;
+        if (__builtin_expect(isSetter, 0)) {
+          if (tid == 0) look.ask(wall_ticks() >= s_setter[2]);
+        }
       }
     };
     auto issue_stage = [&](int t, int tslot) {
@@ -730,34 +731,31 @@ k_persistent_yield(const apk_yield_params) {
       siteDone = s;
       int f = fSeen;
       if (isSetter && tid == 0 && f >= 0) {
+        // Stamped and raised first: what the next one needs (the schedule, from
+        // memory) comes after, or every latency counts it.
         const int64_t now = wall_ticks();
-        if (s_setter[1] == 0) s_setter[1] = now;
-        const long long gBase = s_setter[1];
-        const int nextEv = (int)s_setter[0];
-        // An event is raised only where this block has a later site to see it
-        // from (a flag store shows up in its own samples two or three stages
-        // later): raised at the end of the job's last tile, nobody would be
-        // left to serve it. So at a tile's end it waits unless tasks are left.
-        const int margin = pollStride > 4 ? pollStride : 4;
-        const bool room =
-            S <= 2 * margin || s + margin < S ||
-            TaskQueue(P().next_task, P().M / E::TM, tilesN(), P().num_tasks).any_left();
-        const long long stopAt =
-            gBase + (P().num_events ? P().sched[P().num_events - 1] : 0) + P().stop_after;
-        int ev = nextEv;
-        if (ev < P().num_events) {
-          if (room && now >= gBase + P().sched[ev]) {
+        int ev = (int)s_setter[0];
+        auto due_at = [&]() -> long long {
+          const int n = P().num_events;
+          if (ev < n) return s_setter[1] + P().sched[ev];
+          return P().stop_after > 0 ? s_setter[1] + (n ? P().sched[n - 1] : 0) + P().stop_after
+                                    : LLONG_MAX;
+        };
+        if (s_setter[1] == 0) {
+          s_setter[1] = now;
+          s_setter[2] = due_at();
+        }
+        if (now >= s_setter[2]) {
+          if (ev < P().num_events) {
             P().set_gt[ev] = now;
             set_flag(++ev);
             s_setter[0] = ev;
+            s_setter[2] = due_at();
+          } else {
+            set_flag(-1);  // self-terminating run: no host in the loop
           }
-        } else if (P().stop_after > 0 && now >= stopAt) {
-          set_flag(-1);  // self-terminating run: no host in the loop
         }
-        const long long at = ev < P().num_events ? gBase + P().sched[ev]
-                             : P().stop_after > 0 ? stopAt : LLONG_MAX;
-        s_setter[2] = at;
-        look.next(now >= at);
+        look.ask(now >= s_setter[2]);
       }
       if (f > P().num_events) f = P().num_events;  // never index past the event arrays
       srcKind = AS_IS;

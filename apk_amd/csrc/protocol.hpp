@@ -103,12 +103,6 @@ struct TaskQueue {
   APK_PROTO_FN unsigned list_total(int q) const {
     return (unsigned)(list_begin(q + 1) - list_begin(q)) * passes;
   }
-  // Whether any position is still to be handed out.
-  APK_PROTO_FN bool any_left() const {
-    for (int q = 0; q < APK_QUEUE_XCDS; ++q)
-      if (P::load(&ctr[q]) < list_total(q)) return true;
-    return false;
-  }
   // One caller per block. Returns the next task id, or TQ_NONE when every
   // list is exhausted. `batch` > 1: up to that many consecutive positions of
   // the worker's own list per atomic, while at least 8 batches per worker of
@@ -328,26 +322,24 @@ APK_PROTO_FN int retreat_role(bool continuation, int launch_epoch, int f) {
 // (at_site), and the block leaves its stage loop where it has: leaving drains
 // the software pipeline, which at every site would make the setter's tiles the
 // slowest of the grid. The answer must be the same for every wave, so it is
-// read from block memory: thread 0 looked at the clock at the last site, and
-// looks again now for the next. Two words, used in turn: the one a wave may
-// still be reading at this site is not written before the next site's
-// barrier -- neither by at_site nor, where the block has left the loop with
-// no barrier in between, by next().
+// read from block memory: thread 0 looks at the clock when it samples the flag
+// for the site, in the stage before it (ask). Two words, used in turn: the one
+// a wave may still be reading at this site is not written before the next
+// site's barrier -- neither by ask nor, where the block has left the loop with
+// no barrier in between, by what thread 0 finds there (ask again).
 template <class P>
 struct SetterLook {
   int* due;  // [2], block memory
   int turn;  // uniform: the word that the next site reads
 
-  // Every thread, once per site. `look()` runs in thread 0 only.
-  template <class Look>
-  APK_PROTO_FN bool at_site(bool leader, Look&& look) {
+  // Every thread, once per site.
+  APK_PROTO_FN bool at_site() {
     const bool now = P::uniform(due[turn]) != 0;
     turn ^= 1;
-    if (leader) due[turn] = look();
     return now;
   }
   // Thread 0, between two sites: what the next one reads.
-  APK_PROTO_FN void next(bool v) const { due[turn] = v; }
+  APK_PROTO_FN void ask(bool v) const { due[turn] = v; }
 };
 
 }  // namespace proto

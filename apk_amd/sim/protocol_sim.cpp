@@ -395,12 +395,13 @@ int setter_arm(unsigned seed, int waves, Bug bug) {
     int agreed = -1;
     for (int w : order) {  // one wave from this site's barrier to the next
       auto& l = look[(size_t)w];
-      const bool d = l.at_site(w == 0, [&] { return rng() % 3 == 0; });
+      const bool d = l.at_site();
       if (d && w == 0) {  // out of the loop, with no barrier: an event is raised
         const bool again = rng() % 2 == 0;
-        l.next(again);
+        l.ask(again);
         if (bug == B_DUE_BOTH) due[0] = due[1] = again;
       }
+      if (w == 0) l.ask(rng() % 3 == 0);  // with the sample for the next site
       if (agreed >= 0 && (int)d != agreed) ++split;
       agreed = (int)d;
       left += w == 0 && d;

@@ -284,7 +284,9 @@ typedef struct apk_yield_params {
   int flag_system;             /* 1: flag is host-mapped memory (system scope) */
   int* flag_set;               /* device setter target (block 0) with the same
                                   copies; NULL = none */
-  const long long* sched;      /* [events] cumulative ticks after the setter's first poll */
+  const long long* sched;      /* [events] cumulative ticks after the setter's first poll: an
+                                  event is raised at the setter's (block 0's) first poll site
+                                  that it is due a k-stage (pair) before */
   int num_events;
   long long stop_after;        /* setter stores -1 this many ticks after the
                                   last scheduled event (0 = never) */

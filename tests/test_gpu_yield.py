@@ -321,3 +321,48 @@ def test_mfma128_issue_site_naive_control(torch_gpu, apk, mfma_job):
     say(f"  fired {fired}, checkpoints {_stat(r, apk, apk.ST_CHECKPOINTS)}, in flight "
         f"{_stat(r, apk, apk.ST_INFLIGHT_ALL)}, stale {_stat(r, apk, apk.ST_STALE_ALL)}, "
         f"stale resumed {stale} = corrupted tasks {bad}")
+
+
+@pytest.mark.parametrize("name,kc", [("valu64", 1024), ("mfma128", 1024), ("bf16x256", 1024)])
+def test_event_due_at_the_end_is_raised(torch_gpu, apk, name, kc):
+    """One tile per block and four poll sites in it: an event due between the
+    second and the third is raised, though no task is left and the setter
+    polls only once more."""
+    say(f"{name}: event due in the last tile, k_chunk={kc} of 4096")
+    T, eng = torch_gpu, apk.ENGINES[name]
+    g = apk.geometry(eng)
+    M, N, K = 4 * g.tile_m, 4 * g.tile_n, 4096
+    kind = T.bfloat16 if g.elem_bytes == 2 else T.float32
+    A, B = T.rand(M, K, device="cuda").to(kind), T.rand(N * K, device="cuda").to(kind)
+    C = T.empty(M, N, device="cuda")
+    z = lambda n: T.zeros(n, dtype=T.int64, device="cuda")
+    flag, nxt, run_gt = z(8), z(8), T.zeros(2, dtype=T.int64, device="cuda")
+    sched, set_gt, obs, claim, site = z(1), z(1), z(16), z(1), z(1)
+    u_gt, u_end, uq, exits = z(2), z(1), z(1), z(1)
+    p = apk.YieldParams()
+    p.A, p.B, p.C, p.M, p.N, p.K, p.k_chunk = (A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K,
+                                               kc)
+    p.num_tasks, p.next_task = 16, nxt.data_ptr()
+    p.flag, p.flag_copies, p.flag_set, p.sched = (flag.data_ptr(), 1, flag.data_ptr(),
+                                                  sched.data_ptr())
+    p.num_events, p.poll_every, p.set_gt, p.obs_gt = 1, 1, set_gt.data_ptr(), obs.data_ptr()
+    p.claim, p.claim_site, p.u_gt = claim.data_ptr(), site.data_ptr(), u_gt.data_ptr()
+    p.u_end_max, p.uq_next, p.resume = u_end.data_ptr(), uq.data_ptr(), apk.RESUME_RESTART
+    p.run_gt, p.exit_count = run_gt.data_ptr(), exits.data_ptr()
+
+    def run(at):
+        for t in (flag, nxt, set_gt, obs, claim, site, u_gt, u_end, uq, run_gt, exits):
+            t.zero_()
+        sched.fill_(at)
+        apk.persistent_yield(eng, apk.POLL_CHUNK, False, p, 16,
+                             T.cuda.current_stream().cuda_stream)
+        T.cuda.synchronize()
+        t0, t1 = (int(x) for x in run_gt.cpu())
+        return int(set_gt.cpu()[0]), t0, t1
+
+    run(1 << 40)
+    _, t0, t1 = run(1 << 40)
+    due = (t1 - t0) * 3 // 8  # halfway from the second site to the third
+    raised, s0, s1 = run(due)
+    say(f"  due after {due} ticks of {t1 - t0}, raised after {raised - s0} of {s1 - s0}")
+    assert s0 + due <= raised < s1
