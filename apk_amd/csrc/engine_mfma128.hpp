@@ -423,50 +423,41 @@ struct EngMfma128 {
     mark(verdict, s, seen, least, acc);
   }
   // Stage s in ring slot `slot` enters the pipeline and the two steps of stage
-  // s - 1 leave it; `mid`'s loads are spread over their MFMAs. If stage s - 1
-  // is not FINE, its verdict is returned (uniform), with nothing done. The
-  // verdict is read ahead of the planes, whose reads cover most of its way:
-  // looking for lossy stages costs 4096^3 0.7%, a 256^3 urgent job 14.0 ->
-  // 14.4 us.
+  // s - 1, which must be FINE, leave it; `other`: the first step's blocks from
+  // planes 0 (take_other; its reads also cover the way of that stage's verdict,
+  // read from LDS ahead of them). `mid`'s loads are spread over the MFMAs.
+  // Looking for lossy stages costs 4096^3 0.7%, a 256^3 urgent job 14.0 -> 14.4
+  // us.
   template <class Mid>
-  static __device__ __forceinline__ int stage(char* ring, int slot, int s, Acc& acc, Tail& t,
-                                              int* verdict, Mid&& mid) {
+  static __device__ __forceinline__ void stage(char* ring, int slot, int s, Own& other, Acc& acc,
+                                               Tail& t, int* verdict, Mid&& mid) {
     static_assert(STEPS == 2 && LOADS == 8, "two phases per stage, four loads each");
     const char* abase = ring + slot * STAGE;
     Raw raw;
+    Own odd;
     unsigned seen = 0, unused = 0, least = ~0u;
-    const int v = verdict[(s - 1) & 1];
-    __builtin_amdgcn_sched_barrier(0);
-    Own odd, other;
-    take_other(ring, 0, other);
-    if (const int u = uniform(v)) return u;
     phase<true>(ring, 1, t.own, other, t.raw, odd, unused, acc,
-                   [&](int m) { if (m == 6) load_raw(abase, 0, raw); }, 0, mid);
+                [&](int m) { if (m == 6) load_raw(abase, 0, raw); }, 0, mid);
     lds_sync();
     take_other(ring, 1, other);
     phase<true>(ring, 0, odd, other, raw, t.own, seen, acc,
-                   [&](int m) {
-                     if (m == 6) load_raw(abase, 1, t.raw);
-                     if (m >= 9 && m % 2) watch(t.raw, (m - 9) / 2, least);
-                   },
-                   4, mid);
+                [&](int m) {
+                  if (m == 6) load_raw(abase, 1, t.raw);
+                  if (m >= 9 && m % 2) watch(t.raw, (m - 9) / 2, least);
+                },
+                4, mid);
     mark(verdict, s, seen, least, acc);
-    return FINE;
   }
-  // The two steps left over of stage s, before the accumulators are read;
-  // with nothing done but a barrier if the stage is not FINE.
-  static __device__ __forceinline__ int finish_tail(char* ring, int s, Acc& acc, const Tail& t,
-                                                    const int* verdict) {
+  // The two steps left over of a stage, before the accumulators are read: after
+  // a barrier (every wave's planes), and if the stage is FINE.
+  static __device__ __forceinline__ void finish_tail(char* ring, Acc& acc, const Tail& t) {
     Own odd, other;
     unsigned unused = 0;
-    lds_sync();  // every wave's planes and verdict
-    if (const int u = verdict_of(verdict, s)) return u;
     take_other(ring, 0, other);
     phase<true>(ring, 1, t.own, other, t.raw, odd, unused, acc, [](int) {}, 0, [](int) {});
     lds_sync();
     take_other(ring, 1, other);
     phase<false>(ring, 0, odd, other, t.raw, odd, unused, acc, [](int) {}, 0, [](int) {});
-    return FINE;
   }
 
   // Whether an accumulator of this lane is infinite or NaN.

@@ -364,15 +364,7 @@ k_persistent_yield(const apk_yield_params) {
     // Single stages: the site check comes before the call, and a job that
     // stops there keeps its tail (at issue sites it has run it).
     constexpr bool kStagePipe = PipelinedStages<E>::value;
-    // Whether the tail's stage must be computed with exact products instead
-    // (uniform; after the barrier that follows its call). A block does not
-    // leave at a site then: it steps back, and polls the site when it is
-    // there again.
-    auto steps_back = [&]() -> bool {
-      if constexpr (kStagePipe) return hasTail && E::verdict_of(s_verdict, s - 1) != E::FINE;
-      return false;
-    };
-    int verdict = 0;  // uniform: of the stage that was to be computed
+    int verdict = 0;  // uniform: of the tail's stage, where the block left the loop
 
     // Poll sites are the stages s with s % pollStride == 0; `nextSite` is the
     // next one not yet passed (an urgent tile never reaches one), so a stage
@@ -520,48 +512,29 @@ k_persistent_yield(const apk_yield_params) {
           startHit = true;
         }
       }
-      // One stage per barrier: waits for stage s and polls its site. Whether the
-      // block leaves the loop here (the site found something).
-      auto at_stage = [&]() -> bool {
-        wait_landed<E>();
-        lds_sync();
-        // Poll site: the flag sample for site s has landed with stage s (it
-        // was issued in front of the loads of stage s+1, or of the pair s).
-        // A new generation (or the setter's turn) ends the loop here, before
-        // stage s is computed. With one barrier per stage the flag is read
-        // right after the barrier; with pairs it is read in the engine's
-        // `pre` hook (measured: 10.8% -> 7-9% every-site overhead for the
-        // bf16 engine, while the same placement cost the fp32 engines 1-2%).
-        if constexpr (POLL == APK_POLL_ISSUE && !kStagePipe) {
-          if (!ahead) issue_ahead();
-          ahead = false;
+      // The site that the block re-enters at is not polled again.
+      if (E::GROUP == 1 && s == siteDone && s == nextSite) nextSite += siteStride;
+      // One stage per barrier: polls site s, right after the stage's barrier --
+      // the flag sample for it has landed with the stage (it was issued in
+      // front of the loads of stage s+1, or of the pair s). Returns whether
+      // there is something new (a generation, or the setter's turn): the loop
+      // then ends here, before stage s is computed. With pairs the flag is read
+      // in the engine's `pre` hook (measured: 10.8% -> 7-9% every-site overhead
+      // for the bf16 engine, while the same placement cost the fp32 engines
+      // 1-2%).
+      auto site_news = [&]() -> bool {
+        int f = uniform(flagring[site_flag(slot)]);
+        if (syncPoll) {
+          // The blocks that retreat at the next generation read the flag itself
+          // at the site (one load and one barrier) instead of the sample issued
+          // a stage earlier.
+          if (tid == 0) s_fsync = flag_load(myFlag);
+          lds_sync();
+          f = uniform(s_fsync);
         }
-        if (POLL != APK_POLL_OFF && s == nextSite) {
-          if (s != siteDone) {
-            int f = uniform(flagring[site_flag(slot)]);
-            if (syncPoll) {
-              // The blocks that retreat at the next generation read the
-              // flag itself at the site (one load and one barrier) instead
-              // of the sample issued a stage earlier.
-              if (tid == 0) s_fsync = flag_load(myFlag);
-              lds_sync();
-              f = uniform(s_fsync);
-            }
-            fLatest = f;
-            if (((int)setter_due() | (f != lastSeen)) && !steps_back()) {
-              fSeen = f;
-              atSite = true;
-              if constexpr (!kStagePipe) ahead = POLL == APK_POLL_ISSUE;
-              return true;
-            }
-          }
-          if (!steps_back()) nextSite += siteStride;  // else still to come
-        }
-        if constexpr (POLL == APK_POLL_ISSUE && kStagePipe) {
-          if (!ahead && !steps_back()) issue_ahead();
-          ahead = false;
-        }
-        return false;
+        fLatest = f;
+        fSeen = f;
+        return ((int)setter_due() | (f != lastSeen)) != 0;
       };
       // The hook under stage s's matrix work: stage s+2 (and the sample for a
       // site at s+1) goes out there; its slot held stage s-1, which every wave
@@ -573,45 +546,92 @@ k_persistent_yield(const apk_yield_params) {
         }
       };
       if constexpr (kStagePipe) {
-        // Two loops: see run_split_stages.
+        // Two loops: see run_split_stages. Each has one way out at its top, with
+        // every reason to leave in one condition (more ways out cost register
+        // moves in every stage).
         typename E::Dst d;
-        bool carry = false;  // s + 1 is a site
-        auto mid = [&](int i) { load_ahead(d, carry, i); };
+        auto mid = [&](int i) { load_ahead(d, false, i); };
+        // The sample for a site at s + 1 goes out here, ahead of the stage's
+        // MFMAs: a branch among them keeps the compiler from filling the time
+        // of the first ones.
         auto ahead_of = [&] {
-          carry = s + 1 == nextSite;
+          if (POLL == APK_POLL_ISSUE) {
+            if (!ahead) issue_ahead();
+            ahead = false;
+          } else if (s + 1 == nextSite) {
+            sample(slot_after_next(slot));
+          }
           d = E::stage_dst(wl, ctx, slot_after_next(slot), s + 2, S);
         };
         auto step = [&] {
           slot = next_slot<E>(slot);
           ++s;
         };
-        if (mode == E::SPLIT) {
-          if (!hasTail && !atSite && !at_stage()) {
+        bool news = false;
+        if (!atSite && mode != E::SPLIT) {
+          while (s < S) {
+            wait_landed<E>();
+            lds_sync();
+            const bool site = POLL != APK_POLL_OFF && s == nextSite;
+            if (site) news = site_news();
+            if (news) break;
+            if (site) nextSite += siteStride;
+            ahead_of();
+            E::compute_exact(ring, slot, acc, mid);
+            step();
+          }
+        } else if (!atSite && !hasTail) {
+          wait_landed<E>();
+          lds_sync();
+          const bool site = POLL != APK_POLL_OFF && s == nextSite;
+          if (site) news = site_news();
+          if (!news) {
+            if (site) nextSite += siteStride;
             ahead_of();
             E::enter(ring, slot, s, acc, tail, s_verdict, mid);
             hasTail = true;
             step();
           }
-          while (!atSite && s < S) {
-            if (at_stage()) break;
+        }
+        if (!atSite && !news && mode == E::SPLIT) {
+          while (s < S) {
+            wait_landed<E>();
+            lds_sync();
+            const int v = s_verdict[(s - 1) & 1];
+            __builtin_amdgcn_sched_barrier(0);
+            const bool site = POLL != APK_POLL_OFF && s == nextSite;
+            if (site) news = site_news();
+            typename E::Own other;
+            E::take_other(ring, 0, other);
+            verdict = uniform(v);
+            if ((int)news | verdict) break;
+            if (site) nextSite += siteStride;
             ahead_of();
-            verdict = E::stage(ring, slot, s, acc, tail, s_verdict, mid);
-            if (verdict != E::FINE) break;
-            step();
-          }
-        } else {
-          while (!atSite && s < S) {
-            if (at_stage()) break;
-            ahead_of();
-            E::compute_exact(ring, slot, acc, mid);
+            E::stage(ring, slot, s, other, acc, tail, s_verdict, mid);
             step();
           }
         }
+        // A stage that is not FINE comes first: the block steps back, and polls
+        // the site when it is there again.
+        if (news && verdict == E::FINE) atSite = true;
       }
       while (!kStagePipe && !atSite && s < S) {
         if constexpr (kStagePipe) {
         } else if constexpr (E::GROUP == 1) {
-          if (at_stage()) break;
+          wait_landed<E>();
+          lds_sync();
+          if constexpr (POLL == APK_POLL_ISSUE) {
+            if (!ahead) issue_ahead();
+            ahead = false;
+          }
+          if (POLL != APK_POLL_OFF && s == nextSite) {
+            if (site_news()) {
+              atSite = true;
+              ahead = POLL == APK_POLL_ISSUE;
+              break;
+            }
+            nextSite += siteStride;
+          }
           const bool carry = s + 1 == nextSite;  // s+1 is a site
           const typename E::Dst d = E::stage_dst(wl, ctx, slot_after_next(slot), s + 2, S);
           E::compute(ring, slot, acc, [] { return true; },
@@ -694,35 +714,42 @@ k_persistent_yield(const apk_yield_params) {
       }
       if constexpr (kStagePipe) {
         // At a site the tail waits: a block that goes on keeps it.
-        if ((POLL == APK_POLL_ISSUE || !atSite) && hasTail && verdict == E::FINE)
-          verdict = E::finish_tail(ring, s - 1, acc, tail, s_verdict);
-        if (POLL == APK_POLL_ISSUE || !atSite) hasTail = false;
+        if (POLL == APK_POLL_ISSUE || !atSite) {
+          if (hasTail && verdict == E::FINE) {
+            lds_sync();
+            verdict = E::verdict_of(s_verdict, s - 1);
+          }
+          const bool had = hasTail;
+          hasTail = false;
+          if (verdict == E::LOSSY) {
+            // Back to the tail's stage, still in its slot (its successor's
+            // loads go out once more, to the same place).
+            verdict = E::FINE;
+            mode = E::EXACT_REST;
+            --s;
+            slot = slot_before(slot);
+            srcKind = AS_IS;
+            continue;
+          }
+          bool again = verdict == E::BROKEN;
+          if (!again && had) E::finish_tail(ring, acc, tail);
+          if (!atSite) {
+            if (!again && mode != E::EXACT && E::broken(acc)) s_verdict[2] = 1;
+            wait_vmcnt<0>();  // the refetches past the tile's end have landed
+            lds_sync();       // every wave done with the ring; every sample has landed
+            if (again || (mode != E::EXACT && take_broken<E>(s_verdict))) {
+              verdict = E::FINE;
+              mode = E::EXACT;
+              srcKind = FRESH;
+              s = 0;
+              siteDone = -1;
+              continue;
+            }
+          }
+        }
         if constexpr (POLL == APK_POLL_ISSUE) {
           if (atSite && !ahead) issue_ahead();
           ahead = atSite;
-        }
-        if (verdict == E::LOSSY) {
-          // Back to the tail's stage, still in its slot (its successor's loads
-          // go out once more, to the same place).
-          verdict = E::FINE;
-          mode = E::EXACT_REST;
-          --s;
-          slot = slot_before(slot);
-          srcKind = AS_IS;
-          continue;
-        }
-        if (!atSite) {
-          if (mode != E::EXACT && (verdict == E::BROKEN || E::broken(acc))) s_verdict[2] = 1;
-          wait_vmcnt<0>();  // the refetches past the tile's end have landed
-          lds_sync();       // every wave done with the ring; every sample has landed
-          if (mode != E::EXACT && take_broken<E>(s_verdict)) {
-            verdict = E::FINE;
-            mode = E::EXACT;
-            srcKind = FRESH;
-            s = 0;
-            siteDone = -1;
-            continue;
-          }
         }
       }
       if (!atSite) break;  // the tile is computed
@@ -794,10 +821,12 @@ k_persistent_yield(const apk_yield_params) {
           if (!hasTail) return;
           hasTail = false;
           // (the verdict was FINE when the block left the stage loop)
-          if (P().resume == APK_RESUME_CKPT_FULL)
-            E::finish_tail(ring, s - 1, acc, tail, s_verdict);
-          else
+          if (P().resume == APK_RESUME_CKPT_FULL) {
+            lds_sync();
+            E::finish_tail(ring, acc, tail);
+          } else {
             ckStage = s - 1;
+          }
         }
       };
       // `through`: the slot is read back on another XCD (retreat arm): stores

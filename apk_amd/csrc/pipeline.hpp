@@ -233,14 +233,30 @@ __device__ __forceinline__ void run_split_stages(char* ring, uint32_t wl,
         slot = next_slot<E>(slot);
         if (++s == S) break;
         d = next();
-        v = E::stage(ring, slot, s, acc, tail, verdict, mid);
+        v = verdict[(s - 1) & 1];
+        __builtin_amdgcn_sched_barrier(0);
+        typename E::Own other;
+        E::take_other(ring, 0, other);
+        v = uniform(v);
         if (v != E::FINE) break;
+        E::stage(ring, slot, s, other, acc, tail, verdict, mid);
       }
-      if (v == E::FINE) v = E::finish_tail(ring, S - 1, acc, tail, verdict);
-      if (v == E::LOSSY) {
+      if (v == E::FINE) {
+        lds_sync();
+        v = E::verdict_of(verdict, S - 1);
+      }
+      if (v == E::FINE) {
+        E::finish_tail(ring, acc, tail);
+      } else if (v == E::LOSSY) {
         mode = E::EXACT_REST;
         --s;
         slot = slot_before(slot);
+      } else {
+        mode = E::EXACT;
+        E::zero(acc);
+        wait_vmcnt<0>();
+        lds_sync();
+        continue;
       }
     }
     if (mode != E::SPLIT) {
@@ -250,7 +266,7 @@ __device__ __forceinline__ void run_split_stages(char* ring, uint32_t wl,
         slot = next_slot<E>(slot);
       }
     }
-    if (mode != E::EXACT && (v == E::BROKEN || E::broken(acc))) verdict[2] = 1;
+    if (mode != E::EXACT && E::broken(acc)) verdict[2] = 1;
     wait_vmcnt<0>();
     lds_sync();
     if (mode == E::EXACT || !take_broken<E>(verdict)) return;
