@@ -114,11 +114,13 @@ struct TaskQueue {
     cursor = c;
     return u;
   }
-  // Marks the lists that all the counters, read in one round trip, show
-  // exhausted. A counter only grows, so a list seen exhausted stays so.
+  // Marks the lists that all the counters, read at once, show exhausted. A
+  // counter only grows, so a list seen exhausted stays so. (The line serves
+  // reads no faster than atomics: eight single ones per look took a GEMM of 1.6
+  // tiles per worker, 1024 workers, from 318 to 350 us, two wide ones do not.)
   APK_PROTO_FN void look(QueueCursor& c) const {
     unsigned v[APK_QUEUE_XCDS];
-    for (int i = 0; i < APK_QUEUE_XCDS; ++i) v[i] = P::load(&ctr[i]);
+    P::load_counters(ctr, v);
     for (int i = 0; i < APK_QUEUE_XCDS; ++i)
       if (v[i] >= list_total(i)) c.dead |= 1u << i;
   }

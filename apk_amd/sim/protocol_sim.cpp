@@ -83,6 +83,9 @@ struct HostPlat {
   }
   static unsigned load(const unsigned* p) { return __atomic_load_n(p, kLoadOrder); }
   static int load(const int* p) { return __atomic_load_n(p, kLoadOrder); }
+  static void load_counters(const unsigned* p, unsigned (&v)[APK_QUEUE_XCDS]) {
+    for (int i = 0; i < APK_QUEUE_XCDS; ++i) v[i] = load(p + i);
+  }
   static void store(int* p, int v) { __atomic_store_n(p, v, kStoreOrder); }
 #ifdef APK_SIM_TSAN
   static void acquire() {}
