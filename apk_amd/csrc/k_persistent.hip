@@ -30,7 +30,7 @@ __global__ void __launch_bounds__(E::THREADS) __attribute__((amdgpu_waves_per_eu
 
   const int tilesN = N / E::TN;
   const unsigned numTasks = (unsigned)((M / E::TM) * tilesN);
-  const TaskQueue tq(next_task, M / E::TM, tilesN, numTasks);
+  const proto::TaskQueue<DevPlatWide> tq(next_task, M / E::TM, tilesN, numTasks);
   // Blocks are dealt to the XCDs in turn, so blocks of one list share an L2.
   const int home = tq.home_of((int)(blockIdx.x % APK_QUEUE_XCDS));
   const int nChunks = K / kChunk;

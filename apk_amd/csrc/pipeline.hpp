@@ -22,19 +22,10 @@ struct DevPlat {
   static __device__ __forceinline__ unsigned load(const unsigned* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  // The queue's eight counters, device-coherent: two requests.
   static __device__ __forceinline__ void load_counters(const unsigned* p,
                                                        unsigned (&v)[APK_QUEUE_XCDS]) {
-    static_assert(APK_QUEUE_XCDS == 8, "two 16-byte reads");
-    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-    const buf_rsrc r = make_buf_rsrc(p, APK_QUEUE_XCDS * 4);
-    const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(r, 0, 0, CPOL_SC1);
-    const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(r, 16, 0, CPOL_SC1);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[i] = a[i];
-      v[i + 4] = b[i];
-    }
+    for (int i = 0; i < APK_QUEUE_XCDS; ++i) v[i] = load(p + i);
   }
   static __device__ __forceinline__ int load(const int* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -57,6 +48,25 @@ struct DevPlat {
 };
 
 using TaskQueue = proto::TaskQueue<DevPlat>;
+// The counters with two requests, for grids whose workers all look at about the
+// same time (apk_persistent_gemm; see TaskQueue::look). Not in the preemptible
+// kernels: there the wide reads cost the one-wave bf16 tile, which takes every
+// register, 12% on tasks of 12 stages.
+struct DevPlatWide : DevPlat {
+  static __device__ __forceinline__ void load_counters(const unsigned* p,
+                                                       unsigned (&v)[APK_QUEUE_XCDS]) {
+    static_assert(APK_QUEUE_XCDS == 8, "two 16-byte reads");
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    const buf_rsrc r = make_buf_rsrc(p, APK_QUEUE_XCDS * 4);
+    const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(r, 0, 0, CPOL_SC1);
+    const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(r, 16, 0, CPOL_SC1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[i] = a[i];
+      v[i + 4] = b[i];
+    }
+  }
+};
 using proto::RQ_FULL;
 using proto::RQ_NONE;
 using proto::RQ_STUCK;
