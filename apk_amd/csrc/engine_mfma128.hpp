@@ -12,7 +12,11 @@
 // below 2^-24 of it), accumulated in fp32 by v_mfma_f32_32x32x16_bf16, which
 // rounds once per 8 products where the fp32 instructions round at every one.
 // Error against 64 bits, uniform [-1, 1) operands, K = 256 / 992 / 4096:
-// 2.3e-7 / 4.8e-7 / 1.0e-6 (fp32 chain 2.9e-7 / 5.6e-7 / 1.1e-6).
+// 2.3e-7 / 4.8e-7 / 1.0e-6 (fp32 chain 2.9e-7 / 5.6e-7 / 1.1e-6). Operands
+// spread over 2^-30 .. 2^30, K = 64 / 992: 6.0e-8 / 2.2e-7 (5.1e-8 / 1.7e-7).
+// The three-part split is that of Henry, Tang and Heinecke, "Leveraging the
+// bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations"
+// (2019).
 // What the parts cannot carry is computed with exact fp32 products instead
 // (compute_exact, at the fp32 matrix rate and with the same poll sites):
 //  - from the first k-stage on that holds an operand with bits below 2^-133
@@ -38,8 +42,8 @@
 // the planes (18 instructions per wave and step); without them 1.2 K, at 2.0
 // GHz (the package then limits the clock). Splitting in every wave for itself
 // (no planes, twice the vector work) is no faster, and 6% slower with polls.
-// 4096^3: 970 -> 800 us; 1920x1408x992: 67 -> 53; 8192x8192x4096 with
-// chunk polls: 4130 -> 3430.
+// 4096^3: 970 -> 775-825 us, box by box; 1920x1408x992: 80 -> 54 (with the
+// queue's part); 8192x8192x4096 with chunk polls: 4140 -> 3,280-3,330.
 //
 // LDS layouts (bank-conflict-free):
 //  A stage: 128 rows x 128 B. 16-byte quad q of row r is stored at slot

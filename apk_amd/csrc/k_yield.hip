@@ -813,8 +813,8 @@ k_persistent_yield(const apk_yield_params) {
       // too. Elsewhere the resumed tile computes that stage again, which
       // keeps some 3500 cycles out of the way of the urgent job: flag to
       // urgent start 8.8 -> 7.4 us p50 with accumulator checkpoints, 7.5 ->
-      // 6.2 re-queued, with a 256^3 urgent job on 8192x8192x4096. Blocks that
-      // go on keep the tail: polls at tile boundaries cost 3.7% (5.7%).
+      // 6.0 re-queued, with a 256^3 urgent job on 8192x8192x4096. Blocks that
+      // go on keep the tail.
       int ckStage = s;
       auto settle = [&] {
         if constexpr (kStagePipe) {
@@ -838,7 +838,9 @@ k_persistent_yield(const apk_yield_params) {
         if (observe) before = probe_last_load<E>(ring, newest);
         // drain: every wave's loads landed, then a barrier makes them visible
         // to every thread. naive: no wait and no barrier -- the ring is read
-        // as it stands (no wave writes LDS here; only loads may still land).
+        // as it stands (no wave writes LDS here; only loads may still land). At
+        // the other sites of single stages a FULL checkpoint has run the tail
+        // first, under which they do land: only issue sites show the race there.
         if (drain) {
           wait_vmcnt<0>();
           lds_sync();

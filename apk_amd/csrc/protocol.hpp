@@ -116,8 +116,8 @@ struct TaskQueue {
   }
   // Marks the lists that all the counters, read at once, show exhausted. A
   // counter only grows, so a list seen exhausted stays so. (The line serves
-  // reads no faster than atomics: eight single ones per look took a GEMM of 1.6
-  // tiles per worker, 1024 workers, from 318 to 350 us, two wide ones do not.)
+  // reads no faster than atomics: a GEMM of 1.6 tiles per worker, 1024 workers,
+  // takes 350 us with eight single reads per look, 317 with two wide ones.)
   APK_PROTO_FN void look(QueueCursor& c) const {
     unsigned v[APK_QUEUE_XCDS];
     P::load_counters(ctr, v);
