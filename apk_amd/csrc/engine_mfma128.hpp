@@ -42,7 +42,7 @@
 // the planes (18 instructions per wave and step); without them 1.2 K, at 2.0
 // GHz (the package then limits the clock). Splitting in every wave for itself
 // (no planes, twice the vector work) is no faster, and 6% slower with polls.
-// 4096^3: 970 -> 775-825 us, box by box; 1920x1408x992: 80 -> 54 (with the
+// 4096^3: 970 -> 775-825 us, card by card; 1920x1408x992: 80 -> 54 (with the
 // queue's part); 8192x8192x4096 with chunk polls: 4140 -> 3,280-3,330.
 //
 // LDS layouts (bank-conflict-free):
